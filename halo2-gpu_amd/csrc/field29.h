@@ -55,6 +55,12 @@ struct Fq29Params {
         0x25b68180u, 0x214dc281u, 0x3cb84c67u, 0x0060c89bu };
     static constexpr uint32_t K4M[9] = { 0x21f3f51cu, 0x241182dau, 0x31ca8d3bu, 0x2b548b42u, 0x361765dfu,
         0x2b6d0301u, 0x229b8503u, 0x397098cfu, 0x00c19138u };
+    // 6m likewise; 4m with every limb but the top >= 3 (2^29 - 1), for a subtrahend that is
+    // the limb-wise sum of three normalised values
+    static constexpr uint32_t K6M[9] = { 0x32edefaau, 0x261a4447u, 0x2aafd3d9u, 0x30fed0e4u, 0x212318cfu,
+        0x31238483u, 0x23e94785u, 0x3628e537u, 0x012259d5u };
+    static constexpr uint32_t K4M3[9] = { 0x61f3f51cu, 0x641182d8u, 0x71ca8d39u, 0x6b548b40u, 0x761765ddu,
+        0x6b6d02ffu, 0x629b8501u, 0x797098cdu, 0x00c19136u };
     static constexpr uint32_t ONE[9] = { 0x157ccc21u, 0x141c2758u, 0x185230d3u, 0x014c0419u, 0x0aa36fb9u,
         0x1d4240ceu, 0x11d54c07u, 0x052ac7a8u, 0x000dc836u };
     static constexpr uint32_t TO261[8] = { 0x157ccc21u, 0x4e8384ebu, 0x0ce148c3u, 0xfb90a602u, 0x819caa36u,
@@ -213,9 +219,10 @@ struct F29 {
         return r;
     }
 
-    // (a b + c d) / 2^261 with one reduction for both products: every operand
-    // normalised (limbs < 2^29, values < 2^259), so a column holds at most 27 products
-    // of < 2^58 (< 2^63). Returns normalised limbs of a value < m + (a b + c d) / 2^261.
+    // (a b + c d) / 2^261 with one reduction for both products: a and c normalised, b with
+    // limbs < 1.5 2^30 and d with limbs < 2^30 (values < 2^259), so a column holds at most
+    // 9 (1.5 2^59 + 2^59 + 2^58) = 27 2^59 (< 2^64 with the carry). Returns normalised limbs
+    // of a value < m + (a b + c d) / 2^261.
     __device__ __forceinline__ static F29 mul_sum(const F29& a, const F29& b, const F29& c, const F29& d)
     {
         uint32_t m[9];
@@ -303,6 +310,33 @@ struct F29 {
         for (int i = 0; i < 9; ++i)
             r.l[i] = a.l[i] + P::K4M[i] - b.l[i];
         return r;
+    }
+
+    // a + 6m - b, limb by limb; b normalised with b < 6m (base field only: curve29.h)
+    __device__ __forceinline__ static F29 sub6(const F29& a, const F29& b)
+    {
+        F29 r;
+#pragma unroll
+        for (int i = 0; i < 9; ++i)
+            r.l[i] = a.l[i] + P::K6M[i] - b.l[i];
+        return r;
+    }
+
+    // a + 4m - b, limb by limb; b < 4m with limbs up to 3 (2^29 - 1) (base field only: curve29.h)
+    __device__ __forceinline__ static F29 sub4_wide(const F29& a, const F29& b)
+    {
+        F29 r;
+#pragma unroll
+        for (int i = 0; i < 9; ++i)
+            r.l[i] = a.l[i] + P::K4M3[i] - b.l[i];
+        return r;
+    }
+
+    // normalised r < 2m: is r = 0 mod m, for an r that is hardly ever? One limb decides
+    // nearly always, so the nine-limb comparison sits behind a branch.
+    __device__ __forceinline__ static bool is_zero_mod_rare(const F29& r)
+    {
+        return (r.l[0] == 0 || r.l[0] == P::M[0]) && is_zero_mod(r);
     }
 
     // normalised input of value < 2^261 -> normalised representative < 2m

@@ -969,10 +969,7 @@ __global__ void __launch_bounds__(256) accumulate_kernel(const uint32_t* __restr
         }
         const uint32_t xw[8] = { r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w };
         const uint32_t yw[8] = { r2.x, r2.y, r2.z, r2.w, r3.x, r3.y, r3.z, r3.w };
-        G1A29 q { Fq29::from32(xw), Fq29::from32(yw) };
-        if (ent >> 31)
-            q = q.neg();
-        acc = G1X29::add_affine(acc, q);
+        acc = G1X29::add_affine(acc, G1A29 { Fq29::from32(xw), Fq29::from32(yw) }, (ent >> 31) != 0);
         ent = en;
         r0 = n0;
         r1 = n1;
