@@ -164,7 +164,7 @@ struct G1X29 {
         const Fq29 PP = Fq29::sqr(P);
         if (Fq29::is_zero_mod_rare(PP)) {
             if (Fq29::is_zero_mod(Fq29::reduce_2m(R)))
-                return dbl(p);
+                return dbl_inline(p);
             return inf();
         }
         const Fq29 PPP = Fq29::mul(P, PP);

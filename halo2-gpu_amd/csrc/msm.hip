@@ -23,13 +23,13 @@
 //     bucket split between threads are merged afterwards (one thread for up
 //     to LIGHT pieces, a work-group tree for denser buckets).
 //  5. per window, sum_b b * B_b: running sums over segments of L1 buckets
-//     give pairs (T, S) with  answer = sum T + sum_m m * S_m;  work-group
-//     trees over 256 pairs keep that form (T = T_L + T_R + S_R,
-//     S = 2 (S_L + S_R), S carrying the block size as a weight) until one
-//     pair per window is left.
-//  6. on the host: Horner over the exported window sums (c doublings per
-//     window) and conversion to affine, a serial chain a CPU core finishes
-//     faster than one GPU lane.
+//     give pairs (T, S) with  answer = sum T + L1 sum_m m * S_m;  work-group
+//     trees then sum the T and, for every bit i of m, the S_m with that bit set
+//     (P_i), so sum_m m * S_m = sum_i 2^i P_i: one addition per tree level, four
+//     lanes each (curve29_quad.h), and no doubling. Few buckets skip the segments
+//     (L1 = 1).
+//  6. on the host: Horner over the bits of all windows (the exported T and P_i) and
+//     conversion to affine, a serial chain a CPU core finishes faster than one GPU lane.
 // The result is written as (x, y, 1) or the identity (0, 1, 0) in Montgomery
 // form, the layout of the reference's `cukernel_to_affine` output.
 #include <atomic>
@@ -38,7 +38,7 @@
 #include <vector>
 
 #include "common.h"
-#include "curve29.h"
+#include "curve29_quad.h"
 #include "profile.h"
 #include "scan_u32.h"
 
@@ -53,13 +53,18 @@ constexpr uint32_t R1_PER = 4;
 constexpr uint32_t R1_TILE = R1_THREADS * R1_PER; // points per round-1 tile
 constexpr uint32_t R2_THREADS = 1024;
 constexpr uint32_t R2_CHUNK = 16384; // entries per round-2 chunk (staged in LDS)
-constexpr uint32_t LIGHT = 32; // pieces of a split bucket summed by one thread
+constexpr uint32_t LIGHT = 8; // pieces of a split bucket that one quad sums, more than twice the average bucket's
 constexpr uint32_t HEAVY_THREADS = 256;
 constexpr uint32_t HEAVY_BLOCKS = 512;
 constexpr uint32_t RED_L1 = 16; // at most this many buckets per first-level reduction segment
 constexpr uint64_t RED_THREADS = 1ull << 17; // first-level segments wanted: 2 waves per SIMD
-constexpr uint32_t TREE = 256; // threads (tree leaves) per work-group at later levels
-constexpr uint32_t TREE_K = 2; // pairs folded sequentially into each leaf
+// Up to this many buckets the trees start from the buckets (L1 = 1): they then have lanes to
+// spare for the quads' extra work, and the segments' serial chain is gone. Measured at 2^17
+// and 2^19 buckets as the limit: 2^18 points (294912 buckets) 0.80 and 0.76 ms, a batch of
+// 5 x 2^16 over a table (163840) 0.95 and 0.92 ms; above, segments are the cheaper.
+constexpr uint64_t kTreeOnly = 1ull << 19;
+constexpr uint32_t TREE = 256; // tree leaves per work-group at later levels
+constexpr uint32_t TREE_THREADS = 2 * TREE; // a quad per pair of leaves
 constexpr uint32_t MAX_RED_LEVELS = 8;
 constexpr uint32_t MAX_JOBS = 64; // MSMs in one batched pipeline
 
@@ -93,10 +98,10 @@ struct MsmPlan {
     uint64_t max_chunks; // upper bound on round-2 chunks
     uint32_t S; // sorted entries per accumulation thread
     uint64_t nthr; // upper bound on accumulation threads
-    uint32_t L1; // buckets per first reduction segment
+    uint32_t L1; // buckets per first reduction segment (1: the trees start from the buckets)
     uint32_t nlev; // tree levels after the first
-    uint64_t Mlev[MAX_RED_LEVELS + 1]; // pairs per window: Mlev[0] = B / L1, then / (leaves * K) per level
-    uint32_t Klev[MAX_RED_LEVELS + 1]; // pairs per leaf at level i (i >= 1)
+    uint64_t Mlev[MAX_RED_LEVELS + 1]; // nodes per window: Mlev[0] = B / L1, then / leaves per level
+    uint32_t Qlev[MAX_RED_LEVELS + 1]; // points per node: T, sum of S, and one P per bit of m so far
 };
 
 uint32_t log2_floor(uint64_t n)
@@ -171,6 +176,8 @@ uint32_t plain_msm_width(uint64_t npoints)
     return default_width(2 * npoints, false, GLV_BITS);
 }
 
+uint32_t tree_leaves(uint64_t nodes) { return nodes < TREE ? (uint32_t)nodes : TREE; }
+
 // n points (virtual range), window width c, J MSMs; table_n > 0 selects
 // precomputed bases (each MSM's windows share its bucket set).
 MsmPlan plan_core(uint64_t n, uint32_t c, uint32_t J, uint64_t table_n, uint32_t bits = 255)
@@ -208,19 +215,18 @@ MsmPlan plan_core(uint64_t n, uint32_t c, uint32_t J, uint64_t table_n, uint32_t
     uint32_t l1 = 2;
     while (l1 < RED_L1 && (uint64_t)p.Wb * p.B / (2 * l1) >= RED_THREADS)
         l1 *= 2;
+    if (p.nb <= kTreeOnly)
+        l1 = 1;
     p.L1 = p.B < l1 ? p.B : l1;
     p.Mlev[0] = p.B / p.L1;
-    uint32_t lev = 0;
+    p.Qlev[0] = p.L1 == 1 ? 1 : 2;
+    uint32_t lev = 0, index_bits = 0;
     while (p.Mlev[lev] > 1) {
         const uint64_t Mi = p.Mlev[lev];
         ++lev;
-        if (Mi >= (uint64_t)TREE * TREE_K) {
-            p.Klev[lev] = TREE_K;
-            p.Mlev[lev] = Mi / ((uint64_t)TREE * TREE_K);
-        } else {
-            p.Klev[lev] = Mi > TREE ? (uint32_t)(Mi / TREE) : 1u;
-            p.Mlev[lev] = 1;
-        }
+        index_bits += log2_floor(tree_leaves(Mi));
+        p.Mlev[lev] = Mi / tree_leaves(Mi);
+        p.Qlev[lev] = 2 + index_bits;
     }
     p.nlev = lev;
     return p;
@@ -283,7 +289,7 @@ struct MsmBuffers {
     uint32_t* heavy; // nb queued split buckets + 1 counter
     PointSlot* part; // 2 * nthr partial sums of split buckets
     PointSlot* bsum; // nb
-    PointSlot* red[4]; // (T, S) ping-pong: Wb * Mlev[0] pairs in 0, 1; Wb * Mlev[1] in 2, 3
+    PointSlot* red[2]; // tree nodes, ping-pong: level i in red[i & 1], Wb * Mlev[i] * Qlev[i] points
     void* scan_scratch;
     uint64_t* out; // 12 limbs per MSM
 };
@@ -296,8 +302,12 @@ void carve(WS& ws, const MsmPlan& p, MsmBuffers* b)
     uint64_t scan_n = nh1 + 1;
     if (nh2 + 1 > scan_n)
         scan_n = nh2 + 1;
-    const uint64_t nred = (uint64_t)p.Wb * p.Mlev[0]; // pairs after the first level
-    const uint64_t nred1 = p.nlev ? (uint64_t)p.Wb * p.Mlev[1] : 0; // the most any later level writes
+    uint64_t nred[2] = { 0, 0 };
+    for (uint32_t lev = p.L1 == 1 ? 1 : 0; lev <= p.nlev; ++lev) {
+        const uint64_t m = (uint64_t)p.Wb * p.Mlev[lev] * p.Qlev[lev];
+        if (m > nred[lev & 1])
+            nred[lev & 1] = m;
+    }
     void* v[24];
     int k = 0;
     v[k++] = ws.take(p.table_n ? 0 : 64 * p.pts_count);
@@ -316,10 +326,10 @@ void carve(WS& ws, const MsmPlan& p, MsmBuffers* b)
     v[k++] = ws.take(4 * (p.nb + 1));
     v[k++] = ws.take(128 * 2 * p.nthr);
     v[k++] = ws.take(128 * p.nb);
-    for (int i = 0; i < 4; ++i)
-        v[k++] = ws.take(128 * (i < 2 ? nred : nred1));
+    for (int i = 0; i < 2; ++i)
+        v[k++] = ws.take(128 * nred[i]);
     v[k++] = ws.take(scan_u32_scratch(scan_n));
-    v[k++] = ws.take(128ull * p.Wb); // window sums exported to the host
+    v[k++] = ws.take(128ull * p.Wb * p.Qlev[p.nlev]); // window sums exported to the host
     if (b) {
         k = 0;
         b->pts = (uint8_t*)v[k++];
@@ -338,7 +348,7 @@ void carve(WS& ws, const MsmPlan& p, MsmBuffers* b)
         b->heavy = (uint32_t*)v[k++];
         b->part = (PointSlot*)v[k++];
         b->bsum = (PointSlot*)v[k++];
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 2; ++i)
             b->red[i] = (PointSlot*)v[k++];
         b->scan_scratch = v[k++];
         b->out = (uint64_t*)v[k++];
@@ -985,12 +995,16 @@ __global__ void __launch_bounds__(256) accumulate_kernel(const uint32_t* __restr
 // A bucket split between threads t0 < t1 (t0 holds its first entry, so the
 // bucket did not begin before t0's range) has its pieces in part[2 t0 + 1]
 // and part[2 t] for t0 < t <= t1.
-// Up to LIGHT pieces: one thread sums them; more: queued (heavy[nb] counts).
+// Up to LIGHT pieces more than twice the average bucket's: one quad sums them; more: queued
+// (heavy[nb] counts) for a work-group's tree. (With one lane per bucket and up to 32 pieces
+// each, the longest chain of a 50 003 point MSM took 217 us of its 0.98 ms, now 33; a fixed
+// limit of 8 would queue every bucket of a single 2^20 table MSM, 16 pieces each.)
 __global__ void __launch_bounds__(256) merge_split_kernel(const PointSlot* __restrict__ part,
     const uint32_t* __restrict__ off, uint64_t nb, uint32_t S, PointSlot* __restrict__ bsum,
     uint32_t* __restrict__ heavy)
 {
-    const uint64_t b = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t b = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 2;
+    const uint32_t r = threadIdx.x & 3;
     if (b >= nb)
         return;
     const uint32_t lo = off[b], hi = off[b + 1];
@@ -999,56 +1013,52 @@ __global__ void __launch_bounds__(256) merge_split_kernel(const PointSlot* __res
     const uint32_t t0 = lo / S, t1 = (hi - 1) / S;
     if (t0 == t1)
         return;
-    if (t1 - t0 + 1 > LIGHT) {
-        const uint32_t slot = atomicAdd(&heavy[nb], 1u);
-        heavy[slot] = (uint32_t)b;
+    if (t1 - t0 + 1 > LIGHT + 2 * (uint32_t)(off[nb] / (nb * S))) {
+        if (r == 0) {
+            const uint32_t slot = atomicAdd(&heavy[nb], 1u);
+            heavy[slot] = (uint32_t)b;
+        }
         return;
     }
-    G1X29 acc = G1X29::load(part + 2 * (uint64_t)t0 + 1);
+    Fq29 acc = quad_load(part + 2 * (uint64_t)t0 + 1, r);
     for (uint32_t t = t0 + 1; t <= t1; ++t)
-        acc = G1X29::add(acc, G1X29::load(part + 2 * (uint64_t)t));
-    acc.store(bsum + b);
+        acc = quad_add(acc, quad_load(part + 2 * (uint64_t)t, r), r);
+    quad_store(acc, bsum + b, r);
 }
 
-// one work-group per queued dense bucket: strided partial sums, LDS tree
+// one work-group per queued dense bucket: strided partial sums by quads, LDS tree
 __global__ void __launch_bounds__(HEAVY_THREADS) merge_heavy_kernel(const PointSlot* __restrict__ part,
     const uint32_t* __restrict__ off, uint64_t nb, uint32_t S, const uint32_t* __restrict__ heavy,
     PointSlot* __restrict__ bsum)
 {
-    __shared__ G1X29 sh[HEAVY_THREADS];
+    constexpr uint32_t Q = HEAVY_THREADS / 4;
+    __shared__ PointSlot sh[Q];
+    const uint32_t i = threadIdx.x >> 2, r = threadIdx.x & 3;
     const uint32_t count = heavy[nb];
     for (uint32_t h = blockIdx.x; h < count; h += gridDim.x) {
         const uint32_t b = heavy[h];
         const uint32_t t0 = off[b] / S, t1 = (off[b + 1] - 1) / S;
-        G1X29 acc = G1X29::inf();
-        for (uint32_t q = t0 + threadIdx.x; q <= t1; q += HEAVY_THREADS)
-            acc = G1X29::add(acc, G1X29::load(part + 2 * (uint64_t)q + (q == t0 ? 1 : 0)));
-        sh[threadIdx.x] = acc;
-        for (uint32_t d = HEAVY_THREADS / 2; d > 0; d >>= 1) {
+        Fq29 acc = quad_inf(r);
+        for (uint32_t q = t0 + i; q <= t1; q += Q)
+            acc = quad_add(acc, quad_load(part + 2 * (uint64_t)q + (q == t0 ? 1 : 0), r), r);
+        quad_store(acc, sh + i, r);
+        for (uint32_t d = Q / 2; d > 0; d >>= 1) {
             __syncthreads();
-            if (threadIdx.x < d)
-                sh[threadIdx.x] = G1X29::add(sh[threadIdx.x], sh[threadIdx.x + d]);
+            if (i < d)
+                quad_store(quad_add(quad_load(sh + i, r), quad_load(sh + i + d, r), r), sh + i, r);
         }
         __syncthreads();
-        if (threadIdx.x == 0)
-            sh[0].store(bsum + b);
+        if (threadIdx.x < 8)
+            bsum[b].w[threadIdx.x] = sh[0].w[threadIdx.x];
         __syncthreads();
     }
 }
 
-__device__ __forceinline__ G1X29 dbl_times(G1X29 x, uint32_t k)
-{
-    for (uint32_t i = 0; i < k; ++i)
-        x = G1X29::dbl(x);
-    return x;
-}
-
 // first reduction level: segment m of window w covers buckets (1-based)
-// m*L+1 .. m*L+L.  T = sum_j j * B_{mL+j} (local weights), S = L * sum_j B.
+// m*L+1 .. m*L+L.  T = sum_j j * B_{mL+j} (local weights), S = sum_j B: node t is (T, S).
 // An empty bucket (no entries) is the identity and its bsum slot is not read.
 __global__ void __launch_bounds__(256) reduce_first_kernel(const PointSlot* __restrict__ bsum,
-    const uint32_t* __restrict__ off, uint32_t W, uint32_t B, uint32_t L, uint32_t log_l, uint64_t M,
-    PointSlot* __restrict__ T, PointSlot* __restrict__ S)
+    const uint32_t* __restrict__ off, uint32_t W, uint32_t B, uint32_t L, uint64_t M, PointSlot* __restrict__ nodes)
 {
     const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (uint64_t)W * M)
@@ -1062,94 +1072,74 @@ __global__ void __launch_bounds__(256) reduce_first_kernel(const PointSlot* __re
             run = G1X29::add(run, G1X29::load(bsum + b));
         acc = G1X29::add(acc, run);
     }
-    acc.store(T + t);
-    if (M > 1)
-        dbl_times(run, log_l).store(S + t);
+    acc.store(nodes + 2 * t);
+    run.store(nodes + 2 * t + 1);
 }
 
-// Tree level: work-group g of window w reduces the pairs
-// [g * cnt * K, (g + 1) * cnt * K) of the Mi pairs of that window
-// (answer = sum T + sum_m m S_m, S in units of the current segment size).
-// Leaf i folds K consecutive pairs (local weights 0..K-1, S scaled by K);
-// adjacent blocks of equal size then combine as T = T_L + T_R + S_R,
-// S = 2 (S_L + S_R); after log2(cnt) rounds the block's (T, S) is in the same
-// form with cnt * K times larger segments.
-// The rounds are a chain of dependent point operations, so the two halves of
-// every step run on different waves: threads [0, TREE) form T, threads
-// [TREE, 2 TREE) form S of the same node (2 point operations per round instead
-// of 4). Round d's nodes sit on the first cnt / 2d threads of each half, so the
-// waves with no node left skip the round instead of issuing it with idle lanes.
-__global__ void __launch_bounds__(2 * TREE) reduce_tree_kernel(const PointSlot* __restrict__ Ti,
-    const PointSlot* __restrict__ Si, uint64_t Mi, uint32_t K, uint32_t log_k, PointSlot* __restrict__ To,
-    PointSlot* __restrict__ So)
+// Tree level: work-group (w, g, q) sums point q of the `cnt` nodes [g cnt, (g + 1) cnt) of
+// window w, and for q = 1 (the S of the nodes) also, for every bit i of a node's index in
+// the group, the S of the nodes with that bit set. A node is the points
+// T, S, P_0 .. P_(bits - 1); the group's node has log2(cnt) more P.
+// The tree keeps one array: after the round of distance d the block of 2d leaves that
+// starts at l holds its sum in slot l and its P_i (i <= log2 d) in slot l + 2^i: the right
+// half's sum, which nothing overwrites, is the block's newest P. So each round is one
+// addition deep and has (cnt / 2d) (log2 d + 1) of them, at most 128: a quad each, and the
+// waves without one go to the barrier. (With one lane per addition and the pairs' weights
+// kept by doublings, a round was an addition and a doubling or another addition deep: 256
+// leaves took 125-180 us, now 33.)
+// BUCKETS: the nodes are the buckets themselves (S only, weight m + 1, so T is the sum of S
+// and goes out as both points).
+template <bool BUCKETS>
+__global__ void __launch_bounds__(TREE_THREADS) reduce_tree_kernel(const PointSlot* __restrict__ in,
+    const uint32_t* __restrict__ off, uint64_t Mi, uint32_t cnt, uint32_t Qi, PointSlot* __restrict__ out)
 {
-    __shared__ G1X29 sT[TREE];
-    __shared__ G1X29 sS[TREE];
-    const uint64_t per_blk = Mi >= (uint64_t)TREE * K ? (uint64_t)TREE * K : Mi;
-    const uint64_t Mo = Mi / per_blk;
-    const uint32_t cnt = (uint32_t)(per_blk / K);
-    const uint64_t w = blockIdx.x / Mo, g = blockIdx.x % Mo;
-    const uint64_t base = w * Mi + g * per_blk;
-    const bool s_role = threadIdx.x >= TREE; // whole waves: TREE is a multiple of 64
-    // S node i on thread TREE + (i + 64) mod TREE: the waves of a work-group are dealt
-    // to the CU's 4 SIMDs in turn, so the late rounds' T wave (threads 0..63) and S
-    // wave (threads TREE + 64..) issue on different SIMDs instead of sharing one
-    const uint32_t i = s_role ? (threadIdx.x - TREE + TREE - 64) % TREE : threadIdx.x;
-    const bool keep_s = cnt > 1 || Mo > 1;
-    if (i < cnt) {
-        const uint64_t q0 = base + (uint64_t)i * K;
-        if (!s_role) { // T = sum_j T_j + sum_j j S_j
-            G1X29 a = G1X29::load(Ti + q0 + K - 1), run = G1X29::inf(), acc = G1X29::inf();
-            for (int j = (int)K - 1; j > 0; --j) {
-                run = G1X29::add(run, G1X29::load(Si + q0 + (uint32_t)j));
-                acc = G1X29::add(acc, run);
-                a = G1X29::add(a, G1X29::load(Ti + q0 + (uint32_t)j - 1));
-            }
-            sT[i] = G1X29::add(a, acc);
-        } else if (keep_s) { // S = K sum_j S_j
-            G1X29 run = G1X29::load(Si + q0);
-            for (uint32_t j = 1; j < K; ++j)
-                run = G1X29::add(run, G1X29::load(Si + q0 + j));
-            sS[i] = dbl_times(run, log_k);
-        }
+    __shared__ PointSlot sh[TREE];
+    const uint32_t r = threadIdx.x & 3, quad = threadIdx.x >> 2;
+    constexpr uint32_t quads = TREE_THREADS / 4;
+    const uint32_t q = BUCKETS ? 1 : blockIdx.x % Qi;
+    const uint64_t node = BUCKETS ? blockIdx.x : blockIdx.x / Qi; // w Mo + g
+    const uint64_t leaf0 = node * cnt; // w Mi + g cnt
+    for (uint32_t i = quad; i < cnt; i += quads) {
+        Fq29 x;
+        if (BUCKETS)
+            x = off[leaf0 + i + 1] != off[leaf0 + i] ? quad_load(in + leaf0 + i, r) : quad_inf(r);
+        else
+            x = quad_load(in + (leaf0 + i) * Qi + q, r);
+        quad_store(x, sh + i, r);
     }
-    for (uint32_t d = 1; d < cnt; d <<= 1) {
+    uint32_t bits = 0;
+    for (uint32_t d = 1; d < cnt; d <<= 1, ++bits) {
         __syncthreads();
-        const uint32_t l = i * 2 * d, r = l + d;
-        const bool need_s = 2 * d < cnt || Mo > 1;
-        const bool act = r < cnt && (!s_role || need_s);
-        G1X29 v;
-        if (act) {
-            if (!s_role)
-                v = G1X29::add(G1X29::add(sT[l], sT[r]), sS[r]);
-            else
-                v = G1X29::dbl(G1X29::add(sS[l], sS[r]));
-        }
-        __syncthreads();
-        if (act) {
-            if (!s_role)
-                sT[l] = v;
-            else
-                sS[l] = v;
+        const uint32_t per = q == 1 ? bits + 1 : 1;
+        const uint32_t l = quad / per, j = quad % per;
+        if (l < cnt / (2 * d)) {
+            const uint32_t i = l * 2 * d + (j ? 1u << (j - 1) : 0u);
+            quad_store(quad_add(quad_load(sh + i, r), quad_load(sh + i + d, r), r), sh + i, r);
         }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        sT[0].store(To + blockIdx.x);
-        if (Mo > 1)
-            sS[0].store(So + blockIdx.x);
+    const uint32_t Qo = (BUCKETS ? 2 : Qi) + bits;
+    PointSlot* o = out + node * Qo;
+    const uint32_t k = threadIdx.x >> 3, word = threadIdx.x & 7;
+    if (q != 1) {
+        if (k == 0)
+            o[q].w[word] = sh[0].w[word];
+    } else if (k <= bits) { // S, then the new P after the ones the nodes had
+        o[k ? Qo - bits + k - 1 : 1].w[word] = sh[k ? 1u << (k - 1) : 0].w[word];
+        if (BUCKETS && k == 0)
+            o[0].w[word] = sh[0].w[word];
     }
 }
 
-// The window sums leave the device as XYZZ points in the boundary's 2^256 scale
-// (4 x 32 B each, out[t] for window sum t < Wb): the Horner over windows (a chain
-// of c (W - 1) doublings) and the affine conversion run on the host, where one
+// The windows' points (T, S, P_0, ...) leave the device as XYZZ points in the boundary's
+// 2^256 scale (4 x 32 B each, out[t] for point t < count): the Horner over the bits of all
+// windows (c W doublings) and the affine conversion run on the host, where one
 // core finishes the chain in ~0.1 ms while a single GPU lane needs ~1.5 ms for it.
-__global__ void __launch_bounds__(64) export_windows_kernel(const PointSlot* __restrict__ win, uint32_t Wb,
+__global__ void __launch_bounds__(64) export_windows_kernel(const PointSlot* __restrict__ win, uint32_t count,
     uint64_t* __restrict__ out)
 {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= Wb)
+    if (t >= count)
         return;
     const G1Xyzz x = G1X29::load(win + t).to_xyzz256();
     x.X.store(out + 16ull * t);
@@ -1329,17 +1319,21 @@ HXyzz hx_load(const uint64_t* w)
     return r;
 }
 
-// J results of 96 B ((x, y, 1) or (0, 1, 0), Montgomery) from J x Wj window sums
-// of 128 B: sum over w of 2^(c w) S_w by Horner.
-void host_finalize(const uint64_t* win, uint32_t Wj, uint32_t c, uint32_t J, uint64_t* out)
+// J results of 96 B ((x, y, 1) or (0, 1, 0), Montgomery) from J x Wj windows of Q points of
+// 128 B (T, S, P_0 .. P_(Q - 3)): sum over w of 2^(c w) (T + 2^l1 sum_i 2^i P_i) by Horner
+// over the bits, highest first.
+void host_finalize(const uint64_t* win, uint32_t Wj, uint32_t Q, uint32_t c, uint32_t l1, uint32_t J, uint64_t* out)
 {
     for (uint32_t j = 0; j < J; ++j) {
-        const uint64_t* wj = win + 16ull * Wj * j;
-        HXyzz acc = hx_load(wj + 16ull * (Wj - 1));
-        for (int w = (int)Wj - 2; w >= 0; --w) {
-            for (uint32_t k = 0; k < c; ++k)
+        HXyzz acc {}; // the identity
+        for (int w = (int)Wj - 1; w >= 0; --w) {
+            const uint64_t* pt = win + 16ull * Q * ((uint64_t)Wj * j + (uint32_t)w);
+            for (int bit = (int)c - 1; bit >= 0; --bit) {
                 acc = hx_dbl(acc);
-            acc = hx_add(acc, hx_load(wj + 16ull * w));
+                if (bit >= (int)l1 && bit < (int)(l1 + Q - 2))
+                    acc = hx_add(acc, hx_load(pt + 16ull * (2 + (uint32_t)bit - l1)));
+            }
+            acc = hx_add(acc, hx_load(pt));
         }
         uint64_t* o = out + 12ull * j;
         memset(o, 0, 96);
@@ -1356,25 +1350,26 @@ void host_finalize(const uint64_t* win, uint32_t Wj, uint32_t c, uint32_t J, uin
     }
 }
 
-// Copies the J x Wj window sums of a finished pipeline to the host, waits, and
+// Copies the J x Wj windows' points of a finished pipeline to the host, waits, and
 // writes the J 96-byte results to `h_out`.
-// A single MSM's window sums (at most 64 windows: c >= 4) land in a stack buffer, so the
+// A single MSM's points (W (c + 1) < 255 + 2 W <= 383: c >= 4) land in a stack buffer, so the
 // single-MSM entry points, the scratch-free one included, allocate nothing on the host
-// either; only a batch's J x W sums take a heap buffer.
+// either; only a batch takes a heap buffer when it has more.
 RustError finish_on_host(const MsmPlan& p, const MsmBuffers& b, void* h_out, hipStream_t stream)
 {
-    const uint32_t Wj = p.Wb / p.J;
-    constexpr uint32_t kStackWindows = 64;
-    uint64_t local[16 * kStackWindows];
+    const uint32_t Wj = p.Wb / p.J, Q = p.Qlev[p.nlev];
+    const uint64_t count = (uint64_t)p.Wb * Q;
+    constexpr uint32_t kStackPoints = 384;
+    uint64_t local[16 * kStackPoints];
     std::vector<uint64_t> heap;
     uint64_t* win = local;
-    if (p.Wb > kStackWindows) {
-        heap.resize(16ull * p.Wb);
+    if (count > kStackPoints) {
+        heap.resize(16ull * count);
         win = heap.data();
     }
-    H2_TRY(hipMemcpyAsync(win, b.out, 128ull * p.Wb, hipMemcpyDeviceToHost, stream));
+    H2_TRY(hipMemcpyAsync(win, b.out, 128ull * count, hipMemcpyDeviceToHost, stream));
     H2_TRY(hipStreamSynchronize(stream));
-    host_finalize(win, Wj, p.c, p.J, (uint64_t*)h_out);
+    host_finalize(win, Wj, Q, p.c, log2_floor(p.L1), p.J, (uint64_t*)h_out);
     return ok();
 }
 
@@ -1590,27 +1585,33 @@ RustError msm_device(const MsmPlan& p, const MsmBuffers& b, const Fr* d_scalars,
             b.bsum);
         H2_LAUNCH_CHECK();
         H2_TRY(hipMemsetAsync(b.heavy + p.nb, 0, 4, stream));
-        merge_split_kernel<<<blocks_for(p.nb, T), T, 0, stream>>>(b.part, b.off0, p.nb, p.S, b.bsum, b.heavy);
+        merge_split_kernel<<<blocks_for(4 * p.nb, T), T, 0, stream>>>(b.part, b.off0, p.nb, p.S, b.bsum, b.heavy);
         H2_LAUNCH_CHECK();
         merge_heavy_kernel<<<HEAVY_BLOCKS, HEAVY_THREADS, 0, stream>>>(b.part, b.off0, p.nb, p.S, b.heavy, b.bsum);
         H2_LAUNCH_CHECK();
     }
 
     ProfScope prof_red("msm_reduce", stream);
-    const uint64_t M0 = p.Mlev[0];
-    reduce_first_kernel<<<blocks_for((uint64_t)p.Wb * M0, T), T, 0, stream>>>(b.bsum, b.off0, p.Wb, p.B, p.L1,
-        ilog2(p.L1), M0, b.red[0], b.red[1]);
-    H2_LAUNCH_CHECK();
-    int cur = 0;
+    if (p.L1 > 1) {
+        const uint64_t M0 = p.Mlev[0];
+        reduce_first_kernel<<<blocks_for((uint64_t)p.Wb * M0, T), T, 0, stream>>>(b.bsum, b.off0, p.Wb, p.B, p.L1, M0,
+            b.red[0]);
+        H2_LAUNCH_CHECK();
+    }
     for (uint32_t lev = 1; lev <= p.nlev; ++lev) {
         const uint64_t Mi = p.Mlev[lev - 1];
-        const uint64_t Mo = p.Mlev[lev];
-        reduce_tree_kernel<<<(unsigned)(p.Wb * Mo), 2 * TREE, 0, stream>>>(b.red[2 * cur], b.red[2 * cur + 1], Mi,
-            p.Klev[lev], ilog2(p.Klev[lev]), b.red[2 * (cur ^ 1)], b.red[2 * (cur ^ 1) + 1]);
+        const uint32_t Qi = p.Qlev[lev - 1];
+        const unsigned grid = (unsigned)(p.Wb * p.Mlev[lev] * Qi);
+        if (lev == 1 && p.L1 == 1)
+            reduce_tree_kernel<true><<<grid, TREE_THREADS, 0, stream>>>(b.bsum, b.off0, Mi, tree_leaves(Mi), Qi,
+                b.red[1]);
+        else
+            reduce_tree_kernel<false><<<grid, TREE_THREADS, 0, stream>>>(b.red[(lev - 1) & 1], nullptr, Mi,
+                tree_leaves(Mi), Qi, b.red[lev & 1]);
         H2_LAUNCH_CHECK();
-        cur ^= 1;
     }
-    export_windows_kernel<<<blocks_for(p.Wb, 64), 64, 0, stream>>>(b.red[2 * cur], p.Wb, b.out);
+    const uint32_t count = (uint32_t)(p.Wb * p.Qlev[p.nlev]);
+    export_windows_kernel<<<blocks_for(count, 64), 64, 0, stream>>>(b.red[p.nlev & 1], count, b.out);
     H2_LAUNCH_CHECK();
     return ok();
 }

@@ -507,3 +507,28 @@ def test_kzg_table_width_guard(lib, co):
         assert (fresh.commit_many_device([poly, poly[: 4 * 100]])[0] == ref).all()
     finally:
         autotune.set_msm_widths({})
+
+
+@pytest.mark.parametrize("n,table", [(8, False), (257, False), (1 << 15, False), (1 << 15, True), (1 << 20, True)])
+def test_msm_reduction_of_equal_and_opposite_buckets(lib, co, n, table):
+    """Scalars 1, 2, ..., n on bases that are all G, then G and -G in turn: neighbouring
+    buckets hold equal points, then opposite ones, so the reduction's additions meet the
+    doubling and identity cases at every level; entry sizes with trees alone and with
+    segments before them. 1000 equal scalars more make a bucket of many pieces."""
+    from halo2_amd import device as dv, fields as F, msm
+
+    vals = list(range(1, n + 1)) if n <= 1000 else list(range(1, n - 999)) + [5] * 1000
+    sc = np.zeros((n, 4), dtype=np.uint64)
+    sc[:, 0] = vals
+    d_sc = dv.to_device(co.field_mul(0, sc, np.tile(F.mont_limbs(pow(2, 256, F.R_MOD)), (n, 1))))
+    g = co.g1_generator()[:8].reshape(1, 8)
+    minus = g.copy()
+    minus[0, 4:] = F.mont_limbs(F.P_MOD - F.value_of(g[0, 4:], F.P_MOD), F.P_MOD)
+    for signs in ([1], [1, -1], [1, 1, -1, -1]):
+        rows = np.concatenate([g if s > 0 else minus for s in signs])
+        pts = dv.to_device(np.tile(rows, (-(-n // len(signs)), 1))[:n])
+        total = sum(v * signs[i % len(signs)] for i, v in enumerate(vals)) % F.R_MOD
+        exp = co.g1_mul(co.g1_generator(), F.mont_limbs(total))
+        got = msm.multiexp_precomputed(d_sc, msm.msm_precompute(pts, n), n, n) if table \
+            else msm.multiexp_device_scalars_device_bases(d_sc, pts, n)
+        assert (got == exp).all(), signs
