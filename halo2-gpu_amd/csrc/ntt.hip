@@ -63,6 +63,14 @@ uint64_t sized(uint32_t t, uint32_t log_act, uint64_t in_elems, uint64_t out_ele
     return s.bytes + 4096;
 }
 
+RustError build_tables(Workspace& ws, NttTables& t, uint32_t log_n, const Fr* d_omega, NttTwist tw, NttPost post,
+    const Fr& divisor, hipStream_t stream)
+{
+    const NttTableSpec spec { log_n, d_omega, tw == TWIST_POWERS, divisor, post, divisor };
+    NttTables* out = &t;
+    return ntt_tables_build(&spec, &out, 1, ws, stream);
+}
+
 RustError check_log(const char* who, uint32_t log_act)
 {
     if (log_act < 1 || log_act > NTT_MAX_LOG)
@@ -113,7 +121,7 @@ RustError _halo2_fft_normal(uint32_t ntt_type, uint32_t log_n, const void* input
     kind_params(ntt_type, tw, post);
     Fr div = host_fr(divisor);
     NttTables tabs;
-    e = ntt_tables_build(ws, tabs, log_n, d_omega, tw == TWIST_POWERS, div, stream);
+    e = build_tables(ws, tabs, log_n, d_omega, tw, post, div, stream);
     if (e.code)
         return e;
     NttJob job { data, data };
@@ -155,7 +163,7 @@ RustError _halo2_fft_normal_to_device(uint32_t ntt_type, uint32_t log_n, const v
     kind_params(ntt_type, tw, post);
     Fr div = host_fr(h_divisor);
     NttTables tabs;
-    e = ntt_tables_build(ws, tabs, log_n, (const Fr*)d_omega, tw == TWIST_POWERS, div, stream);
+    e = build_tables(ws, tabs, log_n, (const Fr*)d_omega, tw, post, div, stream);
     if (e.code)
         return e;
     NttJob job { (const Fr*)d_input, (Fr*)d_output };
@@ -186,7 +194,7 @@ RustError _halo2_cosetfft(uint32_t ntt_type, uint32_t log_n, uint32_t extend_log
     H2_TRY(hipMemcpyAsync(din, input, 32 * n, hipMemcpyHostToDevice, stream));
     H2_TRY(hipMemcpyAsync(d_omega, omega, 32, hipMemcpyHostToDevice, stream));
     NttTables tabs;
-    e = ntt_tables_build(ws, tabs, extend_log_n, d_omega, false, Fr::zero(), stream);
+    e = build_tables(ws, tabs, extend_log_n, d_omega, TWIST_ZETA, POST_NONE, Fr::zero(), stream);
     if (e.code)
         return e;
     NttJob job { din, dout };
@@ -251,7 +259,7 @@ static RustError fft_many_impl(const char* who, uint32_t ntt_type, uint32_t num_
     kind_params(ntt_type, tw, post);
     Fr div = host_fr(divisor->ptr);
     NttTables tabs;
-    e = ntt_tables_build(ws, tabs, la, (const Fr*)d_omega, tw == TWIST_POWERS, div, stream);
+    e = build_tables(ws, tabs, la, (const Fr*)d_omega, tw, post, div, stream);
     if (e.code)
         return e;
     if (input_on_device && output_on_device) {
@@ -354,6 +362,8 @@ RustError h2amd_fft_batch_to_device(uint32_t ntt_type, uint32_t count, const uin
     std::vector<uint32_t> owner(count), las(count);
     std::vector<Fr> divs(count);
     std::vector<NttBatchJob> jobs(count);
+    std::vector<NttTableSpec> specs;
+    std::vector<NttTables*> built;
     for (uint32_t i = 0; i < count; ++i) {
         if (log_n[i] == 0 || extend_log_n[i] == 0)
             return fail((int)hipErrorInvalidValue, "%s: log_n and extend_log_n must be >= 1 (job %u)", who, i);
@@ -366,24 +376,26 @@ RustError h2amd_fft_batch_to_device(uint32_t ntt_type, uint32_t count, const uin
                 log_n[i], la);
         las[i] = la;
         divs[i] = host_fr(divisors[i].ptr);
-        // jobs of one size, omega (and coset factor) share their tables
+        // jobs of one size, omega (and coset factor or output scale) share their tables
         owner[i] = i;
         for (uint32_t k = 0; k < i; ++k) {
-            const bool same_c = tw != TWIST_POWERS || !memcmp(divs[k].v, divs[i].v, 32);
+            const bool same_c = (tw != TWIST_POWERS && post == POST_NONE) || !memcmp(divs[k].v, divs[i].v, 32);
             if (las[k] == la && d_omega[k] == d_omega[i] && same_c) {
                 owner[i] = owner[k];
                 break;
             }
         }
         if (owner[i] == i) {
-            e = ntt_tables_build(ws, tabs[i], la, (const Fr*)d_omega[i], tw == TWIST_POWERS, divs[i], stream);
-            if (e.code)
-                return e;
+            specs.push_back(NttTableSpec { la, (const Fr*)d_omega[i], tw == TWIST_POWERS, divs[i], post, divs[i] });
+            built.push_back(&tabs[i]);
         }
         Fr* scr = ntt_plan(la).P == 3 ? (Fr*)ws.take(32ull << la) : nullptr;
         jobs[i] = NttBatchJob { &tabs[owner[i]], la, 1ull << log_n[i], (const Fr*)d_in[i], (Fr*)d_out[i], scr,
             divs[i] };
     }
+    RustError e = ntt_tables_build(specs.data(), built.data(), (int)specs.size(), ws, stream);
+    if (e.code)
+        return e;
     void* d_pass = ws.take(ntt_batch_pass_bytes((int)count));
     if (ws.overflow)
         return fail((int)hipErrorInvalidValue, "%s: workspace of %lu bytes is too small", who,

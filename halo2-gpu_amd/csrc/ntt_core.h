@@ -2,17 +2,19 @@
 //
 // Algorithm: Stockham-ordered four-step decomposition N = R_1 * ... * R_P
 // (P = 1..3 passes, R_p <= 2^12). Pass p reads R_p-point columns with stride
-// N/R_p, runs a radix-2 decimation-in-time sub-FFT of the columns in LDS
-// (bit-reversed load, natural-order result), multiplies by the inter-pass
-// twiddle and writes with the autosort index map, so the output of the last
-// pass is in natural order without a bit-reversal pass. The last pass is
-// in-place safe (it writes exactly the positions it read), so an NTT needs at
-// most one scratch buffer of N elements and none when input and output differ
-// and P <= 2.
+// N/R_p, runs a radix-16 / radix-8 decimation-in-frequency sub-FFT of the columns
+// in LDS (ntt_mfma.h; the digit-reversed result is read back in natural order),
+// multiplies by the inter-pass twiddle and writes with the autosort index map, so
+// the output of the last pass is in natural order without a bit-reversal pass.
+// The last pass is in-place safe (it writes exactly the positions it read), so an
+// NTT needs at most one scratch buffer of N elements and none when input and
+// output differ and P <= 2. Transforms of less than 2^6 points are summed by
+// definition, one thread per output.
 //
 // Twiddles never come from a dense 2^(k-1) table: omega^e = lo[e mod 2^h] *
 // hi[e >> h] with two tables of ~2^(k/2) entries that stay resident in L2, and
-// each pass radix has a table of R/2 entries.
+// every step of a pass but its last has a table of its own (one entry per
+// element of a block).
 #pragma once
 
 #include "common.h"
@@ -39,6 +41,7 @@ struct NttPlan {
 
 static constexpr uint32_t NTT_MAX_LOG_R = 12; // 4096 elements = 128 KiB of LDS per work-group
 static constexpr uint32_t NTT_MAX_LOG = 28;
+static constexpr uint32_t NTT_MATRIX_LOG = 6; // smallest transform that runs in matrix steps (two of radix 8)
 static constexpr int NTT_MAX_BATCH = 32; // polynomials per launch (pointers travel as kernel args)
 
 NttPlan ntt_plan(uint32_t log_n);
@@ -47,18 +50,30 @@ struct NttTables {
     const Fr* tw_lo = nullptr; // omega^i, i < 2^h
     const Fr* tw_hi = nullptr; // omega^(i 2^h)
     uint32_t h = 0;
-    const Fr* twr[3] = { nullptr, nullptr, nullptr }; // omega_{R_p}^x, x < R_p / 2
-    const Fr* c_lo = nullptr; // c^i, i < 2^h
-    const Fr* c_hi = nullptr; // c^(i 2^h)
+    const Fr* twr[3] = { nullptr, nullptr, nullptr }; // a pass's step twiddles (omega^x below NTT_MATRIX_LOG)
+    const uint32_t* unit = nullptr; // exponent of the transform's 16th root (ntt_mfma.h)
+    const uint4* last_matrices = nullptr; // the last step's matrices, output scale included
+    const Fr* c_rows = nullptr; // c^(i N / R_1), i < R_1
+    const Fr* c_cols = nullptr; // c^i, i < N / R_1
 };
 
 // Workspace bytes for the tables of one transform size (+ optional c tables).
 void ntt_tables_size(WorkspaceSizer& ws, uint32_t log_n, bool powers_twist);
 
-// Builds the tables in `ws`. `d_omega` is a device pointer to omega; `c` is the
-// CosetFFT_Part factor (used only with powers_twist).
-RustError ntt_tables_build(Workspace& ws, NttTables& t, uint32_t log_n, const Fr* d_omega, bool powers_twist,
-    const Fr& c, hipStream_t stream);
+// What one transform's tables are made from: `d_omega` is a device pointer to omega, `c` the
+// CosetFFT_Part factor (used only with powers_twist), `scale` the output's factor (POST_SCALE*).
+struct NttTableSpec {
+    uint32_t log_n;
+    const Fr* d_omega;
+    bool powers_twist;
+    Fr c;
+    NttPost post;
+    Fr scale;
+};
+
+// Builds the tables of `count` transforms in `ws`, several transforms' per launch.
+RustError ntt_tables_build(const NttTableSpec* specs, NttTables* const* tables, int count, Workspace& ws,
+    hipStream_t stream);
 
 struct NttJob {
     const Fr* in;

@@ -395,3 +395,46 @@ def test_coeff_to_extended_batch(lib, co, po):
     outs = coeff_to_extended_batch_device(doms, polys)
     for dom, p, o in zip(doms, polys, outs):
         assert bool((dom.coeff_to_extended_many_device([p])[0] == o).all()), f"k={dom.k}"
+
+
+@pytest.mark.parametrize("k", [4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 15, 17, 19, 21])
+def test_matrix_steps_other_roots_and_scales(lib, co, k):
+    """Every radix split of a pass (2^6 .. 2^12 rows: all orders of radix-16 and radix-8
+    steps, 2^5 and below by definition) under roots whose 16th root of unity is another one
+    (omega^u, u odd), with an arbitrary output scale, and icosetFFT (scale and zeta powers on
+    the way out), against the oracle's FFT."""
+    from halo2_amd import device as dv, fields as F, ntt
+
+    n = 1 << k
+    a = rand_fr(co, n, 900 + k)
+    a[0], a[n - 1] = F.limbs(F.R_MOD - 1), 0
+    d = dv.to_device(a)
+    out = dv.empty_u64(4 * n)
+    scale = 0x1234567890ABCDEF << 150
+    for u in (1, 3, -1, 11):
+        w = pow(F.omega(k), u, F.R_MOD)
+        exp = co.fft(a, k, F.mont_limbs(w))
+        ntt.fft_normal_device(ntt.FFT, k, d, out, w, 1)
+        assert (dv.to_host(out) == exp).all(), u
+        scaled = co.scale_inplace(np.array(exp, copy=True), F.mont_limbs(scale))
+        ntt.fft_normal_device(ntt.IFFT, k, d, out, w, scale)
+        assert (dv.to_host(out) == scaled).all(), u
+        if k <= 13:
+            z = [F.ZETA * F.ZETA % F.R_MOD, F.ZETA]  # zeta^-1, zeta^-2
+            ico = co.distribute_powers_zeta(scaled, np.stack([F.mont_limbs(v) for v in z]))
+            assert (ntt.fft_gpu(ntt.ICOSET_FFT, a, k, w, scale) == ico).all(), u
+
+
+@pytest.mark.parametrize("kind", [1, 2, 6])
+def test_batch_of_every_small_size(lib, co, po, kind):
+    """One uneven batch of 2^1 .. 2^14: direct transforms and matrix steps in one launch."""
+    from halo2_amd import device as dv, fields as F, ntt
+
+    ks = list(range(1, 15))
+    ins = [rand_fr(co, 1 << k, 950 + k) for k in ks]
+    c = 0xABCDEF987654321
+    omegas = [F.inv(F.omega(k)) if kind == 2 else F.omega(k) for k in ks]
+    divs = [F.inv(1 << k) if kind == 2 else c for k in ks]
+    outs = ntt.fft_batch_to_device(kind, [dv.to_device(a) for a in ins], ks, ks, omegas, divs)
+    for k, a, o in zip(ks, ins, outs):
+        assert (dv.to_host(o) == _oracle_kind(co, po, kind, a, k, c=c)).all(), k
