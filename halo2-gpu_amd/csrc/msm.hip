@@ -87,6 +87,7 @@ struct MsmPlan {
     bool glv; // scalars split k = k1 + lambda k2: 2 nbase virtual points of 128-bit scalars
     uint64_t pts_count; // bases held in the 2^261 scale: nbase, or 2 nbase with the endomorphism images
     uint32_t J; // MSMs in the pipeline (1 unless batched); each has its own W bucket sets (1 with a table)
+    bool batch; // job tables in the workspace (a batch of one MSM too: its tiles end at its length)
     uint32_t c, W, B;
     uint32_t Wb; // bucket windows: J W, or J when the windows share buckets (precomputed bases)
     uint64_t table_n; // precomputed bases: row stride of the table (0 = plain bases)
@@ -269,6 +270,7 @@ MsmPlan make_batch_plan(const uint64_t* lengths, uint32_t J, uint64_t table_n = 
     p.ntiles = (uint32_t)(nv / R1_TILE);
     p.nbase = nmax;
     p.pts_count = nmax;
+    p.batch = true;
     return p;
 }
 
@@ -311,8 +313,8 @@ void carve(WS& ws, const MsmPlan& p, MsmBuffers* b)
     void* v[24];
     int k = 0;
     v[k++] = ws.take(p.table_n ? 0 : 64 * p.pts_count);
-    v[k++] = ws.take(p.J > 1 ? sizeof(BatchJob) * p.J : 0);
-    v[k++] = ws.take(p.J > 1 ? 4ull * p.ntiles : 0);
+    v[k++] = ws.take(p.batch ? sizeof(BatchJob) * p.J : 0);
+    v[k++] = ws.take(p.batch ? 4ull * p.ntiles : 0);
     v[k++] = ws.take(32 * p.n);
     v[k++] = ws.take(4 * nh1);
     v[k++] = ws.take(4 * (nh1 + 1));
@@ -1532,7 +1534,7 @@ unsigned blocks_for(uint64_t n, unsigned t) { return (unsigned)((n + t - 1) / t)
 uint32_t ilog2(uint32_t x) { return 31 - __builtin_clz(x); }
 
 // Full device pipeline; the window sums land in b.out (device, for finish_on_host). A batch
-// (p.J > 1) has its canonical scalars and job tables in place already and
+// (p.batch) has its canonical scalars and job tables in place already and
 // passes d_scalars = null.
 RustError msm_device(const MsmPlan& p, const MsmBuffers& b, const Fr* d_scalars, const uint8_t* d_points,
     hipStream_t stream)
@@ -1557,8 +1559,8 @@ RustError msm_device(const MsmPlan& p, const MsmBuffers& b, const Fr* d_scalars,
         H2_LAUNCH_CHECK();
         pts = b.pts;
     }
-    SortParams sp { p.n, p.c, p.W, p.FB, p.CB, p.NC, p.ntiles, p.table_n, p.NCj, p.J > 1 ? b.jobs : nullptr,
-        p.J > 1 ? b.tile_job : nullptr };
+    SortParams sp { p.n, p.c, p.W, p.FB, p.CB, p.NC, p.ntiles, p.table_n, p.NCj, p.batch ? b.jobs : nullptr,
+        p.batch ? b.tile_job : nullptr };
     const uint64_t nh1 = (uint64_t)p.NCj * p.ntiles; // every tile counts the bins of its own MSM
     r1_count_kernel<<<p.ntiles, R1_THREADS, 4 * p.NCj, stream>>>(b.canon, sp, b.h1);
     H2_LAUNCH_CHECK();

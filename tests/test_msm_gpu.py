@@ -532,3 +532,28 @@ def test_msm_reduction_of_equal_and_opposite_buckets(lib, co, n, table):
         got = msm.multiexp_precomputed(d_sc, msm.msm_precompute(pts, n), n, n) if table \
             else msm.multiexp_device_scalars_device_bases(d_sc, pts, n)
         assert (got == exp).all(), signs
+
+
+@pytest.mark.parametrize("n", [1, 5, 4095, 4097, 5000])
+def test_msm_batch_of_one(lib, co, n):
+    """A batch of a single MSM whose length is not a whole number of sort tiles, over plain
+    bases and over a table: scratch that held other scalars before must not enter it."""
+    import torch
+
+    from halo2_amd import device as dv, msm
+
+    pts = co.g1_mul_gen(rand_fr(co, n, 31 + n))
+    c = rand_fr(co, n, 32 + n)
+    exp = co.msm(c, pts)
+    d_c, d_pts = dv.to_device(c), dv.to_device(pts)
+    table = msm.msm_precompute(d_pts, n)
+    junk = dv.to_device(rand_fr(co, 1 << 16, 33))
+    for _ in range(2):
+        stale = junk.repeat(16)  # freed right away: the scratch that follows holds its words
+        torch.cuda.synchronize()
+        del stale
+        assert (msm.multiexp_batch_device([d_c], d_pts)[0] == exp).all()
+        stale = junk.repeat(16)
+        torch.cuda.synchronize()
+        del stale
+        assert (msm.multiexp_batch_precomputed([d_c], table, n)[0] == exp).all()
