@@ -74,6 +74,7 @@ constexpr uint32_t MAX_JOBS = 64; // MSMs in one batched pipeline
 struct BatchJob {
     uint64_t voff, n;
     uint32_t tile0, tiles;
+    const Fr* scalars;
 };
 
 // 128-byte slot holding one XYZZ point (four 32-byte coordinates)
@@ -96,6 +97,8 @@ struct MsmPlan {
     uint32_t NCj; // coarse bins per MSM = (W, or 1 for shared buckets) << CB
     uint32_t NC; // coarse bins = J * NCj
     uint32_t ntiles; // round-1 tiles
+    uint32_t groups; // work-groups per round-1 tile, each for wper windows
+    uint32_t wper;
     uint64_t max_chunks; // upper bound on round-2 chunks
     uint32_t S; // sorted entries per accumulation thread
     uint64_t nthr; // upper bound on accumulation threads
@@ -177,6 +180,18 @@ uint32_t plain_msm_width(uint64_t npoints)
     return default_width(2 * npoints, false, GLV_BITS);
 }
 
+// Few tiles leave compute units idle while each tile goes through its windows one after the
+// other (~4 us each), so a tile's windows are dealt to several work-groups, up to ~2 per compute
+// unit: round 1 of a 1500 point MSM 137 -> 37 us, of 50 003 points 109 -> 46.
+void set_tiles(MsmPlan& p, uint32_t ntiles)
+{
+    p.ntiles = ntiles;
+    uint32_t groups = ntiles ? 512 / ntiles : 1;
+    groups = groups < 1 ? 1 : groups > p.W ? p.W : groups;
+    p.wper = (p.W + groups - 1) / groups;
+    p.groups = (p.W + p.wper - 1) / p.wper;
+}
+
 uint32_t tree_leaves(uint64_t nodes) { return nodes < TREE ? (uint32_t)nodes : TREE; }
 
 // n points (virtual range), window width c, J MSMs; table_n > 0 selects
@@ -198,14 +213,18 @@ MsmPlan plan_core(uint64_t n, uint32_t c, uint32_t J, uint64_t table_n, uint32_t
     p.CB = p.c - 1 - p.FB;
     p.NCj = (table_n ? 1u : p.W) << p.CB;
     p.NC = J * p.NCj;
-    p.ntiles = (uint32_t)((n + R1_TILE - 1) / R1_TILE);
+    set_tiles(p, (uint32_t)((n + R1_TILE - 1) / R1_TILE));
     const uint64_t work = n * p.W;
     p.max_chunks = work / R2_CHUNK + p.NC;
     // ~2^20 accumulation threads, 16..128 entries each: longer runs than buckets
-    // split fewer buckets between threads (less merging) and still fill the chip
+    // split fewer buckets between threads (less merging) and still fill the chip.
+    // Work that gives less than a wave per SIMD even at 8 entries takes 8: its time is
+    // one thread's chain (1500 points 365 -> 341 us, three 2^12 table MSMs 377 -> 338;
+    // five of 2^16 would go from 0.89 to 0.99 ms)
     uint64_t s = work >> 20;
-    if (s < 16)
-        s = 16;
+    const uint64_t least = work < (8ull << 16) ? 8 : 16;
+    if (s < least)
+        s = least;
     if (s > 128)
         s = 128;
     p.S = (uint32_t)s;
@@ -267,7 +286,7 @@ MsmPlan make_batch_plan(const uint64_t* lengths, uint32_t J, uint64_t table_n = 
         c = 16;
     MsmPlan p = plan_core(nv ? nv : 1, c, J, table_n);
     p.n = nv;
-    p.ntiles = (uint32_t)(nv / R1_TILE);
+    set_tiles(p, (uint32_t)(nv / R1_TILE));
     p.nbase = nmax;
     p.pts_count = nmax;
     p.batch = true;
@@ -296,10 +315,14 @@ struct MsmBuffers {
     uint64_t* out; // 12 limbs per MSM
 };
 
+// round-1 counters: every tile counts the bins of its own MSM; where the windows share the
+// bins (a table), each of its work-groups does
+uint64_t r1_counts(const MsmPlan& p) { return (uint64_t)p.NCj * p.ntiles * (p.table_n ? p.groups : 1); }
+
 template <class WS>
 void carve(WS& ws, const MsmPlan& p, MsmBuffers* b)
 {
-    const uint64_t nh1 = (uint64_t)p.NCj * p.ntiles; // every tile counts the bins of its own MSM
+    const uint64_t nh1 = r1_counts(p);
     const uint64_t nh2 = p.max_chunks << p.FB;
     uint64_t scan_n = nh1 + 1;
     if (nh2 + 1 > scan_n)
@@ -383,6 +406,17 @@ __global__ void to_canonical_kernel(const Fr* __restrict__ scal, uint32_t* __res
         return;
     Fr v = Fr::from_mont(Fr::load(scal + i));
     v.store(canon + 8 * i);
+}
+
+// the same for every MSM of a batch: block (x, y) is quarter y of round-1 tile x
+__global__ void __launch_bounds__(1024) to_canonical_batch_kernel(const BatchJob* __restrict__ jobs,
+    const uint32_t* __restrict__ tile_job, uint32_t* __restrict__ canon)
+{
+    const BatchJob jb = jobs[tile_job[blockIdx.x]];
+    const uint64_t v = (uint64_t)blockIdx.x * R1_TILE + blockIdx.y * 1024u + threadIdx.x; // virtual index
+    if (v - jb.voff >= jb.n)
+        return;
+    Fr::from_mont(Fr::load(jb.scalars + (v - jb.voff))).store(canon + 8 * v);
 }
 
 // bases -> 2^261 scale (x * 2^261 = Montgomery product of x * 2^256 and 2^261);
@@ -554,11 +588,14 @@ struct SortParams {
     uint32_t NCj; // coarse bins per MSM
     const BatchJob* jobs; // null for a single MSM
     const uint32_t* tile_job;
+    uint32_t wper; // windows per work-group of a tile
+    uint32_t cols; // counter columns per tile: the work-groups of a table's tile have their own
 };
 
 // The MSM a round-1 tile belongs to: its virtual point range and tile range.
 // The round-1 histogram h1 is job-major, then bin-major, then tile: job j's
-// bin b of its tile t sits at NCj * tile0 + b * tiles + (t - tile0).
+// bin b of its tile t sits at NCj * tile0 + b * tiles + (t - tile0), with `cols` tiles in
+// the place of each (t cols + work-group) where the work-groups of a tile share the bins.
 struct TileRange {
     uint64_t v0, vend;
     uint32_t tile0, tiles;
@@ -567,14 +604,29 @@ struct TileRange {
 __device__ __forceinline__ TileRange tile_range(const SortParams& sp, uint32_t tile)
 {
     if (!sp.jobs)
-        return TileRange { 0, sp.n, 0, sp.ntiles };
+        return TileRange { 0, sp.n, 0, sp.ntiles * sp.cols };
     const BatchJob jb = sp.jobs[sp.tile_job[tile]];
-    return TileRange { jb.voff, jb.voff + jb.n, jb.tile0, jb.tiles };
+    return TileRange { jb.voff, jb.voff + jb.n, jb.tile0 * sp.cols, jb.tiles * sp.cols };
 }
 
-__device__ __forceinline__ uint64_t h1_index(const SortParams& sp, const TileRange& r, uint32_t b, uint32_t tile)
+__device__ __forceinline__ uint64_t h1_index(const SortParams& sp, const TileRange& r, uint32_t b, uint32_t col)
 {
-    return (uint64_t)sp.NCj * r.tile0 + (uint64_t)b * r.tiles + (tile - r.tile0);
+    return (uint64_t)sp.NCj * r.tile0 + (uint64_t)b * r.tiles + (col - r.tile0);
+}
+
+// The windows [w0, w1) of this work-group, its counter column and the bins [b0, b1) it fills
+struct R1Group {
+    uint32_t w0, w1, col, b0, b1;
+};
+__device__ __forceinline__ R1Group r1_group(const SortParams& sp)
+{
+    R1Group g;
+    g.w0 = blockIdx.y * sp.wper;
+    g.w1 = g.w0 + sp.wper < sp.W ? g.w0 + sp.wper : sp.W;
+    g.col = blockIdx.x * sp.cols + (sp.cols > 1 ? blockIdx.y : 0u);
+    g.b0 = sp.table_n ? 0u : g.w0 << sp.CB;
+    g.b1 = sp.table_n ? sp.NCj : g.w1 << sp.CB;
+    return g;
 }
 
 // Round 1, pass 1: per tile of R1_TILE points, LDS histogram over the coarse
@@ -583,9 +635,10 @@ __device__ __forceinline__ uint64_t h1_index(const SortParams& sp, const TileRan
 __global__ void __launch_bounds__(R1_THREADS) r1_count_kernel(const uint32_t* __restrict__ canon, SortParams sp,
     uint32_t* __restrict__ h1)
 {
-    extern __shared__ uint32_t hist[];
+    extern __shared__ uint32_t hist[]; // bins [b0, b1)
     const TileRange tr = tile_range(sp, blockIdx.x);
-    for (uint32_t i = threadIdx.x; i < sp.NCj; i += R1_THREADS)
+    const R1Group gr = r1_group(sp);
+    for (uint32_t i = threadIdx.x; i < gr.b1 - gr.b0; i += R1_THREADS)
         hist[i] = 0;
     __syncthreads();
     const uint64_t p0 = (uint64_t)blockIdx.x * R1_TILE;
@@ -598,17 +651,17 @@ __global__ void __launch_bounds__(R1_THREADS) r1_count_kernel(const uint32_t* __
         for (int q = 0; q < 8; ++q)
             s[q] = canon[8 * i + q];
         uint32_t carry = 0;
-        for (uint32_t w = 0; w < sp.W; ++w) {
+        for (uint32_t w = 0; w < gr.w1; ++w) {
             const int32_t d = next_digit(s, w, sp.c, carry);
-            if (d != 0) {
+            if (d != 0 && w >= gr.w0) {
                 const uint32_t bi = (uint32_t)(d < 0 ? -d : d) - 1u;
-                atomicAdd(&hist[(sp.table_n ? 0u : w << sp.CB) + (bi >> sp.FB)], 1u);
+                atomicAdd(&hist[(sp.table_n ? 0u : (w - gr.w0) << sp.CB) + (bi >> sp.FB)], 1u);
             }
         }
     }
     __syncthreads();
-    for (uint32_t b = threadIdx.x; b < sp.NCj; b += R1_THREADS)
-        h1[h1_index(sp, tr, b, blockIdx.x)] = hist[b];
+    for (uint32_t b = gr.b0 + threadIdx.x; b < gr.b1; b += R1_THREADS)
+        h1[h1_index(sp, tr, b, gr.col)] = hist[b - gr.b0];
 }
 
 // Round 1, pass 2: the same tile places its entries at the scanned offsets.
@@ -634,8 +687,9 @@ __global__ void __launch_bounds__(R1_THREADS) r1_scatter_kernel(const uint32_t* 
     uint16_t* sbin = (uint16_t*)(stage + R1_TILE); // the bin of each staged entry
     __shared__ uint32_t wsum[R1_THREADS / 64];
     const TileRange tr = tile_range(sp, blockIdx.x);
-    for (uint32_t b = threadIdx.x; b < sp.NCj; b += R1_THREADS)
-        cursor[b] = h1off[h1_index(sp, tr, b, blockIdx.x)];
+    const R1Group gr = r1_group(sp);
+    for (uint32_t b = gr.b0 + threadIdx.x; b < gr.b1; b += R1_THREADS)
+        cursor[b] = h1off[h1_index(sp, tr, b, gr.col)];
     const uint32_t fmask = (1u << sp.FB) - 1u;
     const uint64_t p0 = (uint64_t)blockIdx.x * R1_TILE;
     uint32_t s[R1_PER][8];
@@ -649,7 +703,12 @@ __global__ void __launch_bounds__(R1_THREADS) r1_scatter_kernel(const uint32_t* 
             s[k][q] = i < tr.vend ? canon[8 * i + q] : 0u; // a zero scalar has only zero digits
     }
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (uint32_t w = 0; w < sp.W; ++w) {
+    for (uint32_t w = 0; w < gr.w0; ++w) { // the carries into this work-group's first window
+#pragma unroll
+        for (uint32_t k = 0; k < R1_PER; ++k)
+            (void)next_digit(s[k], w, sp.c, carry[k]);
+    }
+    for (uint32_t w = gr.w0; w < gr.w1; ++w) {
         for (uint32_t b = threadIdx.x; b <= BW; b += R1_THREADS)
             base[b] = 0;
         __syncthreads();
@@ -731,18 +790,19 @@ __global__ void __launch_bounds__(R1_THREADS) r1_scatter_kernel(const uint32_t* 
 __device__ __forceinline__ uint32_t bin_lo(const uint32_t* __restrict__ h1off, const SortParams& sp, uint32_t g)
 {
     if (!sp.jobs)
-        return h1off[(uint64_t)g * sp.ntiles];
+        return h1off[(uint64_t)g * sp.ntiles * sp.cols];
     if (g >= sp.NC)
-        return h1off[(uint64_t)sp.NCj * sp.ntiles];
+        return h1off[(uint64_t)sp.NCj * sp.ntiles * sp.cols];
     const BatchJob jb = sp.jobs[g / sp.NCj];
-    return h1off[(uint64_t)sp.NCj * jb.tile0 + (uint64_t)(g % sp.NCj) * jb.tiles];
+    return h1off[((uint64_t)sp.NCj * jb.tile0 + (uint64_t)(g % sp.NCj) * jb.tiles) * sp.cols];
 }
 
 // One work-group: bin boundaries from the round-1 scan, and the number of
 // round-2 chunks per bin (at least one, so every bucket offset gets written).
 // Thread t owns the contiguous bins [t * per, (t + 1) * per).
 __global__ void __launch_bounds__(1024) bin_info_kernel(const uint32_t* __restrict__ h1off, SortParams sp,
-    uint32_t* __restrict__ bin_start, uint32_t* __restrict__ chunk_base, uint32_t* __restrict__ off0_end)
+    uint32_t* __restrict__ bin_start, uint32_t* __restrict__ chunk_base, uint32_t* __restrict__ off0_end,
+    uint32_t* __restrict__ heavy_count)
 {
     __shared__ uint32_t s[1024];
     const uint32_t per = (sp.NC + 1023) / 1024;
@@ -782,6 +842,7 @@ __global__ void __launch_bounds__(1024) bin_info_kernel(const uint32_t* __restri
         bin_start[sp.NC] = total;
         chunk_base[sp.NC] = s[1023];
         *off0_end = total;
+        *heavy_count = 0; // for the merges
     }
 }
 
@@ -1560,16 +1621,16 @@ RustError msm_device(const MsmPlan& p, const MsmBuffers& b, const Fr* d_scalars,
         pts = b.pts;
     }
     SortParams sp { p.n, p.c, p.W, p.FB, p.CB, p.NC, p.ntiles, p.table_n, p.NCj, p.batch ? b.jobs : nullptr,
-        p.batch ? b.tile_job : nullptr };
-    const uint64_t nh1 = (uint64_t)p.NCj * p.ntiles; // every tile counts the bins of its own MSM
-    r1_count_kernel<<<p.ntiles, R1_THREADS, 4 * p.NCj, stream>>>(b.canon, sp, b.h1);
+        p.batch ? b.tile_job : nullptr, p.wper, p.table_n ? p.groups : 1u };
+    const dim3 r1_grid(p.ntiles, p.groups);
+    r1_count_kernel<<<r1_grid, R1_THREADS, 4 * p.NCj, stream>>>(b.canon, sp, b.h1);
     H2_LAUNCH_CHECK();
-    RustError e = scan_u32_exclusive(b.h1, b.h1off, nh1, b.scan_scratch, stream);
+    RustError e = scan_u32_exclusive(b.h1, b.h1off, r1_counts(p), b.scan_scratch, stream);
     if (e.code)
         return e;
-    r1_scatter_kernel<<<p.ntiles, R1_THREADS, r1_scatter_lds(p.NCj, p.CB), stream>>>(b.canon, sp, b.h1off, b.kv1);
+    r1_scatter_kernel<<<r1_grid, R1_THREADS, r1_scatter_lds(p.NCj, p.CB), stream>>>(b.canon, sp, b.h1off, b.kv1);
     H2_LAUNCH_CHECK();
-    bin_info_kernel<<<1, 1024, 0, stream>>>(b.h1off, sp, b.bin_start, b.chunk_base, b.off0 + p.nb);
+    bin_info_kernel<<<1, 1024, 0, stream>>>(b.h1off, sp, b.bin_start, b.chunk_base, b.off0 + p.nb, b.heavy + p.nb);
     H2_LAUNCH_CHECK();
     r2_count_kernel<<<(unsigned)p.max_chunks, R2_THREADS, 0, stream>>>(b.kv1, sp, b.bin_start, b.chunk_base, b.h2);
     H2_LAUNCH_CHECK();
@@ -1586,7 +1647,6 @@ RustError msm_device(const MsmPlan& p, const MsmBuffers& b, const Fr* d_scalars,
         accumulate_kernel<<<blocks_for(p.nthr, T), T, 0, stream>>>(b.entries, pts, b.off0, p.nb, p.S, b.part,
             b.bsum);
         H2_LAUNCH_CHECK();
-        H2_TRY(hipMemsetAsync(b.heavy + p.nb, 0, 4, stream));
         merge_split_kernel<<<blocks_for(4 * p.nb, T), T, 0, stream>>>(b.part, b.off0, p.nb, p.S, b.bsum, b.heavy);
         H2_LAUNCH_CHECK();
         merge_heavy_kernel<<<HEAVY_BLOCKS, HEAVY_THREADS, 0, stream>>>(b.part, b.off0, p.nb, p.S, b.heavy, b.bsum);
@@ -1889,20 +1949,16 @@ static RustError batch_entry(const char* who, const void* const* d_scalars, cons
     uint64_t voff = 0;
     for (uint32_t j = 0; j < count; ++j) {
         const uint64_t span = align_tile(lengths[j]);
-        jobs[j] = BatchJob { voff, lengths[j], (uint32_t)(voff / R1_TILE), (uint32_t)(span / R1_TILE) };
+        jobs[j] = BatchJob { voff, lengths[j], (uint32_t)(voff / R1_TILE), (uint32_t)(span / R1_TILE),
+            (const Fr*)d_scalars[j] };
         for (uint32_t t = 0; t < jobs[j].tiles; ++t)
             tile_job[jobs[j].tile0 + t] = j;
         voff += span;
     }
     H2_TRY(hipMemcpyAsync(b.jobs, jobs.data(), sizeof(BatchJob) * count, hipMemcpyHostToDevice, stream));
     H2_TRY(hipMemcpyAsync(b.tile_job, tile_job.data(), 4ull * p.ntiles, hipMemcpyHostToDevice, stream));
-    for (uint32_t j = 0; j < count; ++j) {
-        if (lengths[j] == 0)
-            continue;
-        to_canonical_kernel<<<blocks_for(lengths[j], 256), 256, 0, stream>>>((const Fr*)d_scalars[j],
-            b.canon + 8 * jobs[j].voff, lengths[j]);
-        H2_LAUNCH_CHECK();
-    }
+    to_canonical_batch_kernel<<<dim3(p.ntiles, R1_TILE / 1024), 1024, 0, stream>>>(b.jobs, b.tile_job, b.canon);
+    H2_LAUNCH_CHECK();
     RustError e = msm_device(p, b, nullptr, (const uint8_t*)d_bases, stream);
     if (e.code)
         return e;

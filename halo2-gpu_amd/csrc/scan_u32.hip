@@ -10,8 +10,9 @@ constexpr unsigned kThreads = 1024;
 constexpr unsigned kPer = 4;
 constexpr unsigned kTile = kThreads * kPer;
 
+// `total`: where the whole sum goes when one block scans everything (null otherwise)
 __global__ void __launch_bounds__(kThreads) scan_tile_kernel(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
-    uint64_t n, uint32_t* __restrict__ block_sums)
+    uint64_t n, uint32_t* __restrict__ block_sums, uint32_t* __restrict__ total)
 {
     __shared__ uint32_t s[kThreads];
     const uint64_t base = (uint64_t)blockIdx.x * kTile + (uint64_t)threadIdx.x * kPer;
@@ -37,21 +38,25 @@ __global__ void __launch_bounds__(kThreads) scan_tile_kernel(const uint32_t* __r
             out[base + k] = run;
         run += v[k];
     }
-    if (threadIdx.x == kThreads - 1)
+    if (threadIdx.x == kThreads - 1) {
         block_sums[blockIdx.x] = s[kThreads - 1];
+        if (total)
+            *total = s[kThreads - 1];
+    }
 }
 
-__global__ void add_block_kernel(uint32_t* __restrict__ out, uint64_t n, const uint32_t* __restrict__ block_pre)
+// the last thread's element also gives the whole sum (`total`, if not null): its scanned value
+// plus its input
+__global__ void add_block_kernel(const uint32_t* __restrict__ in, uint32_t* __restrict__ out, uint64_t n,
+    const uint32_t* __restrict__ block_pre, uint32_t* __restrict__ total)
 {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n)
-        out[i] += block_pre[i / kTile];
-}
-
-__global__ void write_total_kernel(uint32_t* out, uint64_t n, const uint32_t* in)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0)
-        out[n] = (n ? out[n - 1] + in[n - 1] : 0u);
+    if (i >= n)
+        return;
+    const uint32_t v = out[i] + block_pre[i / kTile];
+    out[i] = v;
+    if (total && i == n - 1)
+        *total = v + in[i];
 }
 
 } // namespace
@@ -67,19 +72,20 @@ uint64_t scan_u32_scratch(uint64_t n)
     return bytes + 256;
 }
 
-static RustError scan_rec(const uint32_t* in, uint32_t* out, uint64_t n, uint8_t* scratch, hipStream_t stream)
+static RustError scan_rec(const uint32_t* in, uint32_t* out, uint64_t n, uint8_t* scratch, uint32_t* total,
+    hipStream_t stream)
 {
     const uint64_t nb = (n + kTile - 1) / kTile;
     uint32_t* sums = (uint32_t*)scratch;
     uint32_t* sums_pre = (uint32_t*)(scratch + align_up(4 * (nb + 1), 256));
     uint8_t* next = scratch + 2 * align_up(4 * (nb + 1), 256);
-    scan_tile_kernel<<<(unsigned)nb, kThreads, 0, stream>>>(in, out, n, sums);
+    scan_tile_kernel<<<(unsigned)nb, kThreads, 0, stream>>>(in, out, n, sums, nb == 1 ? total : nullptr);
     H2_LAUNCH_CHECK();
     if (nb > 1) {
-        RustError e = scan_rec(sums, sums_pre, nb, next, stream);
+        RustError e = scan_rec(sums, sums_pre, nb, next, nullptr, stream);
         if (e.code)
             return e;
-        add_block_kernel<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(out, n, sums_pre);
+        add_block_kernel<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(in, out, n, sums_pre, total);
         H2_LAUNCH_CHECK();
     }
     return ok();
@@ -91,12 +97,7 @@ RustError scan_u32_exclusive(const uint32_t* in, uint32_t* out, uint64_t n, void
         H2_TRY(hipMemsetAsync(out, 0, 4, stream));
         return ok();
     }
-    RustError e = scan_rec(in, out, n, (uint8_t*)scratch, stream);
-    if (e.code)
-        return e;
-    write_total_kernel<<<1, 64, 0, stream>>>(out, n, in);
-    H2_LAUNCH_CHECK();
-    return ok();
+    return scan_rec(in, out, n, (uint8_t*)scratch, out + n, stream);
 }
 
 } // namespace h2
