@@ -7,8 +7,8 @@
 //   (one table occurrence consumed); the leftover table multiset, ascending,
 //   fills the remaining rows from the last one backwards; rows [U, n) are zero.
 //
-// Sorting: 256-bit canonical keys, merge sort — a tile of 2048 keys is sorted
-// in LDS (8 keys per thread sorted in registers, then 8 merge rounds), then
+// Sorting: 256-bit canonical keys, merge sort — a tile of 8192 keys is sorted
+// in LDS by 51-bit windows of the keys (tile_sort_kernel), then
 // global merge passes, each work-group merging one 2048-key output tile found
 // by a merge-path split. Both arrays (input, table) are sorted by the same
 // launches (grid y). Then: not-head flags over the sorted input, leftover flags
@@ -24,7 +24,8 @@ using namespace h2;
 namespace {
 
 constexpr unsigned kThreads = 256; // element-wise kernels
-constexpr unsigned kTile = 2048; // keys per sorted tile and per merge work-group, 64 KB of LDS
+constexpr unsigned kTile = 2048; // keys per merge work-group, 64 KB of LDS
+constexpr unsigned kSortTile = 8192; // keys per sorted tile: 64 KB of windows, 16 KB of indices
 
 struct Key {
     uint64_t w[4]; // canonical value, little-endian 64-bit words
@@ -93,15 +94,6 @@ __device__ __forceinline__ Fr fr_from_key(const Key& k)
     return v;
 }
 
-__device__ __forceinline__ void cmp_swap(Key& a, Key& b)
-{
-    if (key_lt(b, a)) {
-        const Key t = a;
-        a = b;
-        b = t;
-    }
-}
-
 // Number of elements taken from A among the first `diag` outputs of the
 // stable merge of A (length na) and B (length nb); ties go to A.
 template <class GetA, class GetB>
@@ -141,52 +133,169 @@ __device__ __forceinline__ void merge_run(const Key* A, uint32_t na, const Key* 
     }
 }
 
-// Sorts each 2048-key tile of keys[y * stride + (0, U)) into out: eight keys
-// per thread sorted in registers, then eight merge rounds in LDS.
-constexpr unsigned kSortThreads = 256;
-constexpr unsigned kSortPer = kTile / kSortThreads;
+// Sorts each 8192-key tile of keys[y * stride + (0, U)) into out.
+//
+// What is sorted is not the 32-byte keys but 64-bit words of 51 key bits and the key's 13-bit
+// place in the tile, four times less to move through LDS and registers; the keys themselves
+// are read where they lie and written once, in order. The 51 bits are the window below the
+// highest bit in which the tile's keys differ. If no lower bit exists the words order the
+// keys completely; otherwise neighbours that agree in the window are compared, and only if
+// two of them differ (2^-26 a tile for uniform keys) the tile is sorted again by all its
+// windows, lowest first (the place in the current order keeps each round stable).
+// Words are sorted 8 per thread in registers, then in ten merge rounds.
+// 2^20 rows of two columns: 213 us with keys as the words and 2048 a tile, now 85, and two
+// merge passes of 38 us less.
+constexpr unsigned kSortThreads = 1024;
+constexpr unsigned kSortPer = kSortTile / kSortThreads;
+constexpr unsigned kIndexBits = 13;
+constexpr unsigned kWindow = 64 - kIndexBits;
+constexpr uint32_t kIndexMask = kSortTile - 1;
 
-__global__ void __launch_bounds__(kSortThreads) tile_sort_kernel(const Key* __restrict__ keys,
-    Key* __restrict__ out, uint64_t U, uint64_t stride)
+// bits [shift, shift + 51) of a key in memory
+__device__ __forceinline__ uint64_t key_window(const Key* p, uint32_t shift)
 {
-    __shared__ Key sh[kTile];
-    const Key* src = keys + blockIdx.y * stride;
-    Key* dst = out + blockIdx.y * stride;
-    const uint64_t base = (uint64_t)blockIdx.x * kTile;
-    const uint32_t t = threadIdx.x;
-    for (uint32_t k = t; k < kTile; k += kSortThreads)
-        sh[k] = base + k < U ? key_load(src + base + k) : key_max();
+    const uint32_t q = shift >> 6, sh = shift & 63;
+    uint64_t v = p->w[q] >> sh;
+    if (sh && q < 3)
+        v |= p->w[q + 1] << (64 - sh);
+    return v & ((1ull << kWindow) - 1);
+}
+
+// sorts sh[0, kSortTile): all the words are different
+__device__ __forceinline__ void sort_words(uint64_t* sh)
+{
+    const uint32_t d = threadIdx.x * kSortPer;
+    uint64_t r[kSortPer];
     __syncthreads();
-    Key r[kSortPer];
 #pragma unroll
     for (unsigned k = 0; k < kSortPer; ++k)
-        r[k] = sh[t * kSortPer + k];
-    // odd-even transposition sort of the thread's keys in registers
+        r[k] = sh[d + k];
+    // odd-even transposition sort of the thread's words in registers
 #pragma unroll
     for (unsigned phase = 0; phase < kSortPer; ++phase) {
 #pragma unroll
-        for (unsigned k = phase & 1; k + 1 < kSortPer; k += 2)
-            cmp_swap(r[k], r[k + 1]);
+        for (unsigned k = phase & 1; k + 1 < kSortPer; k += 2) {
+            const uint64_t a = r[k], b = r[k + 1];
+            r[k] = a < b ? a : b;
+            r[k + 1] = a < b ? b : a;
+        }
     }
-    __syncthreads();
-#pragma unroll
-    for (unsigned k = 0; k < kSortPer; ++k)
-        sh[t * kSortPer + k] = r[k];
-    __syncthreads();
-    for (uint32_t w = kSortPer; w < kTile; w <<= 1) {
-        const uint32_t d = t * kSortPer;
-        const uint32_t p = d / (2 * w);
-        const Key* A = sh + p * 2 * w;
-        merge_run<kSortPer>(A, w, A + w, w, d - p * 2 * w, r);
+    for (uint32_t w = kSortPer; w < kSortTile; w <<= 1) {
         __syncthreads();
 #pragma unroll
         for (unsigned k = 0; k < kSortPer; ++k)
             sh[d + k] = r[k];
         __syncthreads();
+        const uint32_t p = d & ~(2 * w - 1), diag = d - p;
+        const uint64_t* A = sh + p;
+        const uint64_t* B = A + w;
+        uint32_t lo = diag > w ? diag - w : 0, hi = diag < w ? diag : w;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (A[mid] < B[diag - 1 - mid])
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        uint32_t i = lo, j = diag - lo;
+        uint64_t a = i < w ? A[i] : ~0ull, b = j < w ? B[j] : ~0ull;
+#pragma unroll
+        for (unsigned k = 0; k < kSortPer; ++k) {
+            const bool takeA = j >= w || (i < w && a < b);
+            r[k] = takeA ? a : b;
+            if (takeA) {
+                ++i;
+                a = i < w ? A[i] : ~0ull;
+            } else {
+                ++j;
+                b = j < w ? B[j] : ~0ull;
+            }
+        }
     }
-    for (uint32_t k = t; k < kTile; k += kSortThreads)
-        if (base + k < U)
-            key_store(dst + base + k, sh[k]);
+    __syncthreads();
+#pragma unroll
+    for (unsigned k = 0; k < kSortPer; ++k)
+        sh[d + k] = r[k];
+    __syncthreads();
+}
+
+__global__ void __launch_bounds__(kSortThreads) tile_sort_kernel(const Key* __restrict__ keys,
+    Key* __restrict__ out, uint64_t U, uint64_t stride)
+{
+    __shared__ uint64_t sh[kSortTile];
+    __shared__ uint16_t perm[kSortTile];
+    __shared__ unsigned long long differ[4];
+    __shared__ uint32_t tie;
+    const uint64_t base = (uint64_t)blockIdx.x * kSortTile;
+    const Key* src = keys + blockIdx.y * stride + base;
+    Key* dst = out + blockIdx.y * stride + base;
+    const uint32_t count = U - base < kSortTile ? (uint32_t)(U - base) : kSortTile;
+    const uint32_t t = threadIdx.x;
+    if (t < 4)
+        differ[t] = 0;
+    if (t == 0)
+        tie = 0;
+    __syncthreads();
+    const Key first = key_load(src);
+    uint64_t x[4] = { 0, 0, 0, 0 };
+    for (uint32_t k = t; k < count; k += kSortThreads) {
+        const Key v = key_load(src + k);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            x[q] |= v.w[q] ^ first.w[q];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        for (int d = 32; d; d >>= 1)
+            x[q] |= __shfl_xor(x[q], d, 64);
+        if ((t & 63) == 0 && x[q])
+            atomicOr(&differ[q], (unsigned long long)x[q]);
+    }
+    __syncthreads();
+    uint32_t bits = 0; // the keys differ in bits below this one only
+    for (int q = 3; q >= 0 && !bits; --q)
+        if (differ[q])
+            bits = 64 * q + 64 - __builtin_clzll(differ[q]);
+    const uint32_t shift = bits > kWindow ? bits - kWindow : 0;
+    // padding sorts last: its words have every window bit set, and its places are past the keys'
+    for (uint32_t k = t; k < kSortTile; k += kSortThreads)
+        sh[k] = ((k < count ? key_window(src + k, shift) : (1ull << kWindow) - 1) << kIndexBits) | k;
+    sort_words(sh);
+    if (shift) {
+        for (uint32_t k = t; k + 1 < count; k += kSortThreads) {
+            const uint64_t a = sh[k], b = sh[k + 1];
+            if ((a ^ b) >> kIndexBits == 0
+                && !key_eq(key_load(src + (a & kIndexMask)), key_load(src + (b & kIndexMask))))
+                tie = 1;
+        }
+    }
+    __syncthreads();
+    if (tie) { // the same for the whole work-group
+        for (uint32_t k = t; k < kSortTile; k += kSortThreads)
+            perm[k] = (uint16_t)k;
+        for (uint32_t lo = 0; lo < bits; lo += kWindow) {
+            __syncthreads();
+            for (uint32_t k = t; k < kSortTile; k += kSortThreads) {
+                const uint32_t i = perm[k];
+                sh[k] = ((i < count ? key_window(src + i, lo) : (1ull << kWindow) - 1) << kIndexBits) | k;
+            }
+            sort_words(sh);
+            uint16_t next[kSortPer];
+#pragma unroll
+            for (unsigned k = 0; k < kSortPer; ++k)
+                next[k] = perm[sh[t + k * kSortThreads] & kIndexMask];
+            __syncthreads();
+#pragma unroll
+            for (unsigned k = 0; k < kSortPer; ++k)
+                perm[t + k * kSortThreads] = next[k];
+        }
+        __syncthreads();
+        for (uint32_t k = t; k < count; k += kSortThreads)
+            key_store(dst + k, key_load(src + perm[k]));
+        return;
+    }
+    for (uint32_t k = t; k < count; k += kSortThreads)
+        key_store(dst + k, key_load(src + (sh[k] & kIndexMask)));
 }
 
 // Geometry of output tile `tile` in a merge pass over runs of length w: the
@@ -433,10 +542,10 @@ RustError _halo2_permute_expression_pair(const void* d_compressed_input, const v
             (const Fr*)d_compressed_table, b.keys[0], U, U);
         H2_LAUNCH_CHECK();
         const unsigned tiles = blocks_for(U, kTile);
-        tile_sort_kernel<<<dim3(tiles, 2), kSortThreads, 0, stream>>>(b.keys[0], b.keys[1], U, U);
+        tile_sort_kernel<<<dim3(blocks_for(U, kSortTile), 2), kSortThreads, 0, stream>>>(b.keys[0], b.keys[1], U, U);
         H2_LAUNCH_CHECK();
         int cur = 1;
-        for (uint64_t w = kTile; w < U; w <<= 1) {
+        for (uint64_t w = kSortTile; w < U; w <<= 1) {
             run_split_kernel<<<blocks_for(4ull * tiles * 64, 256), 256, 0, stream>>>(b.keys[cur], b.splits, U, U, w,
                 tiles);
             H2_LAUNCH_CHECK();

@@ -88,3 +88,31 @@ def test_lookup_product_mirrors(lib, co, free_bytes):
     assert (lookup_product_gpu(pi, pt, ci, ct, beta, gamma, free_bytes=free_bytes) == exp).all()
     got = lookup_product_device(*(dv.to_device(x) for x in (pi, pt, ci, ct)), beta, gamma)
     assert (dv.to_host(got) == exp).all()
+
+
+@pytest.mark.parametrize("U", [2, 63, 8191, 8192, 8193, 3 * 8192 + 1])
+@pytest.mark.parametrize("pattern", ["low_and_high", "window", "top"])
+def test_permute_sort_windows(lib, co, U, pattern):
+    """Columns whose keys a tile cannot order by one 51-bit window: they differ in high bits
+    and, where those agree, in low ones only (every window of the tile is needed); or exactly
+    in the bits of one window; or only in the top word; around the 8192-key tile."""
+    from halo2_amd import device as dv
+    from halo2_amd.fields import R_MOD, mont_limbs
+    from halo2_amd.lookup import permute_expression_pair_device
+
+    rng = np.random.default_rng(U)
+    small = [int(v) for v in rng.integers(0, 97, U)]
+    high = [int(v) for v in rng.integers(0, 5, U)]
+    if pattern == "low_and_high":
+        vals = [(h << 250) + (s << 100) + (h ^ s) for h, s in zip(high, small)]
+    elif pattern == "window":
+        vals = [s << 60 for s in small]
+    else:
+        vals = [(R_MOD - 1) - (s << 195) for s in small]
+    table = np.stack([mont_limbs(v % R_MOD) for v in vals])
+    inp = table[rng.integers(0, U, U)]
+    exp_i, exp_t = co.permute_expression_pair(inp, table, U, U)
+    d_pi, d_pt = dv.empty_u64(4 * U), dv.empty_u64(4 * U)
+    permute_expression_pair_device(dv.to_device(inp), dv.to_device(table), d_pi, d_pt, U, U)
+    assert (dv.to_host(d_pi) == exp_i).all()
+    assert (dv.to_host(d_pt) == exp_t).all()
