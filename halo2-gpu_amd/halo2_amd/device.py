@@ -58,7 +58,8 @@ def ptr(t: torch.Tensor) -> int:
 
 
 def stream() -> int:
-    return int(torch.cuda.current_stream().cuda_stream)
+    """The current stream's handle, without the Stream object around it (5 us of every launch)."""
+    return int(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
 
 
 def sync() -> None:

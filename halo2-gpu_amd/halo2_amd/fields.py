@@ -18,15 +18,15 @@ ROOT_OF_UNITY = pow(GENERATOR, (R_MOD - 1) >> TWO_ADICITY, R_MOD)
 ZETA = 0x30644E72E131A029048B6E193FD84104CC37A73FEC2BC5E9B8CA0B2D36636F23
 DELTA = pow(GENERATOR, 1 << TWO_ADICITY, R_MOD)
 MONT = 1 << 256
+_MONT_INV = {R_MOD: pow(MONT, -1, R_MOD), P_MOD: pow(MONT, -1, P_MOD)}
 
 
 def limbs(x: int) -> np.ndarray:
-    return np.array([(x >> (64 * i)) & 0xFFFFFFFFFFFFFFFF for i in range(4)], dtype=np.uint64)
+    return np.frombuffer(bytearray((x & (MONT - 1)).to_bytes(32, "little")), dtype=np.uint64)
 
 
 def from_limbs(a) -> int:
-    a = np.asarray(a, dtype=np.uint64).reshape(-1)
-    return sum(int(w) << (64 * i) for i, w in enumerate(a[:4]))
+    return int.from_bytes(np.asarray(a, dtype=np.uint64).reshape(-1)[:4].tobytes(), "little")
 
 
 def mont(x: int, m: int = R_MOD) -> int:
@@ -34,7 +34,8 @@ def mont(x: int, m: int = R_MOD) -> int:
 
 
 def unmont(x: int, m: int = R_MOD) -> int:
-    return x * pow(MONT, -1, m) % m
+    inv = _MONT_INV.get(m)  # the inverse itself takes 8 us, 58 times a proof
+    return x * (pow(MONT, -1, m) if inv is None else inv) % m
 
 
 def mont_limbs(x: int, m: int = R_MOD) -> np.ndarray:
