@@ -54,183 +54,174 @@ __device__ __forceinline__ void mac96(uint64_t& acc, uint32_t& c2, uint32_t x, u
         : "v"(x), "v"(y));
 }
 
-// x^-1 mod m (P::M, odd, < 2^254) for 0 < x < m, both as 8 little-endian 32-bit limbs:
-// the binary extended GCD in Pornin's batched form ("Optimized Binary GCD for Modular
-// Inversion", 2020, Algorithm 2 with k = 32). The state is a, b (a = x, b = m) and u, v
-// with a = u x and b = v x (mod m) up to a known power of 2. Each of 17 outer rounds runs
-// 31 binary-GCD steps (halve the even one; when a is odd, swap so that a >= b and subtract)
-// on 64-bit images of a and b (their low 31 bits, exact, which fix every parity, and the
-// top 33 bits of the longer one, for the comparisons), recording the steps as a 2x2 matrix
-// (f0 g0; f1 g1) with |f| + |g| <= 2^31. The matrix is then applied once to the full
-// values: a, b <- (f0 a + g0 b) / 2^31, (f1 a + g1 b) / 2^31 (exact; a negative result is
-// negated with its row), and u, v <- f0 u + g0 v, f1 u + g1 v, each reduced mod m by one
-// Montgomery step of 2^32. 17 x 31 = 527 >= 2 x 254 - 1 steps leave b = gcd = 1 and
-// v = x^-1 2^(527 - 544); the final 17 doublings mod m remove the factor. Variable time
-// (the data is public): ~17 x 31 cheap 64-bit steps and 68 short multi-precision
-// products, against ~700 full-width steps of the plain binary algorithm.
+// m (P::M) in 30-bit limbs
 template <class P>
+__host__ __device__ constexpr int32_t modulus30(int i)
+{
+    const int q = 30 * i / 32, s = 30 * i % 32;
+    const uint64_t w = (uint64_t)(q < 8 ? P::M[q < 8 ? q : 7] : 0u)
+        | (uint64_t)(q + 1 < 8 ? P::M[q + 1 < 8 ? q + 1 : 7] : 0u) << 32;
+    return (int32_t)((w >> s) & 0x3fffffffu);
+}
+
+// x^-1 mod m (P::M, odd, < 2^254) for 0 < x < m, both as 8 little-endian 32-bit limbs, by
+// division steps (Bernstein and Yang, "Fast constant-time gcd computation and modular
+// inversion", 2019, in the form that starts at delta = 1/2). One step on (delta, f, g), f odd:
+//   delta > 0 and g odd: (1 - delta, g, (g - f) / 2)
+//   otherwise:           (1 + delta, f, (g + (g mod 2) f) / 2)
+// It looks at parities only, so 30 steps depend on the low 32 bits of f and g; they are
+// collected in a matrix (u v; q r), |u| + |v| and |q| + |r| <= 2^30, and (f, g) <- matrix (f, g)
+// / 2^30 (exact) and (d, e) <- matrix (d, e) / 2^30 mod m (a multiple of m below 2^29 m in
+// magnitude makes it exact) keep f = d x and g = e x (mod m). At g = 0, f = +-1 and
+// x^-1 = +-d. 590 steps (20 rounds) reach it for inputs below 2^256; the loop's own limit of 25 is
+// what bounds it. |d|, |e| grow by at most m / 2 a round.
+//
+// Within a round several steps are taken at once: with theta = delta - 1/2, the trailing zeros
+// of g are that many steps at once, and as long as theta < 0 the steps only add f to g, so
+// w = -g / f mod 2^k clears k <= -theta bits by one multiple of f. When theta >= 0 and g is
+// odd, f and g are exchanged (g' = -f, theta' = -theta - 1), and the step is one of adding.
+// Variable time: the data is public.
+//
+// ONE: a single lane of the wave is active, so that the steps are held in scalar registers and
+// their branches are scalar ones. What bounds that use is the chain of one lane: ~5 scalar
+// instructions a step in the rounds and ~90 multiply-adds after each. Against 31 plain steps of
+// the binary gcd on 64-bit images a round, the inversion of 128 totals (products.hip) takes
+// 77 us instead of 127.
+template <class P, bool ONE = false>
 __host__ __device__ inline void inv_mod_plain(const uint32_t (&x)[8], uint32_t (&out)[8])
 {
-    uint32_t a[8], b[8], u[8], v[8];
-    for (int i = 0; i < 8; ++i) {
-        a[i] = x[i];
-        b[i] = P::M[i];
-        u[i] = i == 0 ? 1u : 0u;
-        v[i] = 0;
+    constexpr int32_t M30 = 0x3fffffff;
+    auto uniform = [](uint32_t t) -> uint32_t {
+#ifdef __HIP_DEVICE_COMPILE__
+        if constexpr (ONE)
+            return (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
+#endif
+        return t;
+    };
+    int32_t f[9], g[9], d[9], e[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        const int q = 30 * i / 32, s = 30 * i % 32;
+        const uint64_t w = (uint64_t)x[q] | (uint64_t)(q + 1 < 8 ? x[q + 1 < 8 ? q + 1 : 7] : 0u) << 32;
+        f[i] = modulus30<P>(i);
+        g[i] = (int32_t)((w >> s) & M30);
+        d[i] = 0;
+        e[i] = i == 0 ? 1 : 0;
     }
-    auto bitlen = [](const uint32_t (&w)[8]) -> int {
-        for (int i = 7; i >= 0; --i)
-            if (w[i])
-                return 32 * i + 32 - __builtin_clz(w[i]);
-        return 0;
-    };
-    // bits [s, s + 33) of w (s >= 31; limbs past the top are zero)
-    auto top33 = [](const uint32_t (&w)[8], int s) -> uint64_t {
-        const int q = s >> 5, sh = s & 31;
-        const uint64_t w0 = q < 8 ? w[q] : 0, w1 = q + 1 < 8 ? w[q + 1] : 0, w2 = q + 2 < 8 ? w[q + 2] : 0;
-        uint64_t r = ((w1 << 32) | w0) >> sh;
-        if (sh)
-            r |= w2 << (64 - sh);
-        return r & ((1ull << 33) - 1);
-    };
-    // r = (f p + g q) as a signed 288-bit value in 9 limbs (two's complement), p, q < 2^256
-    auto lincomb = [](const uint32_t (&p)[8], const uint32_t (&q)[8], int64_t f, int64_t g, uint32_t (&r)[9]) {
-        const uint64_t fa = (uint64_t)(f < 0 ? -f : f), ga = (uint64_t)(g < 0 ? -g : g); // <= 2^31
-        uint64_t cp = 0, cq = 0;
-        int64_t c = 0;
-        for (int i = 0; i < 9; ++i) {
-            uint64_t tp = cp, tq = cq;
-            if (i < 8) {
-                tp += (uint64_t)p[i] * fa;
-                tq += (uint64_t)q[i] * ga;
+    int theta = 0;
+    for (int round = 0; round < 25; ++round) {
+        int32_t any = 0;
+#pragma unroll
+        for (int i = 0; i < 9; ++i)
+            any |= g[i];
+        if (uniform((uint32_t)any) == 0)
+            break;
+        uint32_t fl = uniform((uint32_t)f[0] | (uint32_t)f[1] << 30);
+        uint32_t gl = uniform((uint32_t)g[0] | (uint32_t)g[1] << 30);
+        uint32_t u = 1, v = 0, q = 0, r = 1; // two's complement, |.| <= 2^30
+        int left = 30;
+        for (;;) {
+            const int z = __builtin_ctz(gl | 1u << left);
+            gl >>= z;
+            u <<= z;
+            v <<= z;
+            theta += z;
+            left -= z;
+            if (left == 0)
+                break;
+            if (theta >= 0) {
+                uint32_t t = fl;
+                fl = gl;
+                gl = 0u - t;
+                t = u;
+                u = q;
+                q = 0u - t;
+                t = v;
+                v = r;
+                r = 0u - t;
+                theta = -theta - 1;
             }
-            const int64_t lp = (int64_t)(uint32_t)tp, lq = (int64_t)(uint32_t)tq;
-            cp = tp >> 32;
-            cq = tq >> 32;
-            const int64_t t = (f < 0 ? -lp : lp) + (g < 0 ? -lq : lq) + c;
-            r[i] = (uint32_t)t;
-            c = t >> 32; // arithmetic
+            int k = -theta < left ? -theta : left;
+            k = k < 6 ? k : 6;
+            // f (2 - f^2) = 1 / f mod 2^6 (f is its own inverse mod 2^3)
+            const uint32_t w = (gl * fl * (fl * fl - 2u)) & ((1u << k) - 1u);
+            gl += fl * w;
+            q += u * w;
+            r += v * w;
         }
-    };
-    // a, b update: r / 2^31 with its sign; returns true when r was negative (then |r| / 2^31)
-    auto shift31 = [](uint32_t (&r)[9], uint32_t (&o)[8]) -> bool {
-        const bool neg = (int32_t)r[8] < 0;
-        if (neg) { // two's complement negation
-            uint64_t c = 1;
-            for (int i = 0; i < 9; ++i) {
-                const uint64_t t = (uint64_t)(uint32_t)~r[i] + c;
-                r[i] = (uint32_t)t;
-                c = t >> 32;
-            }
+        const int32_t ui = (int32_t)u, vi = (int32_t)v, qi = (int32_t)q, ri = (int32_t)r;
+        int64_t cf = (int64_t)ui * f[0] + (int64_t)vi * g[0];
+        int64_t cg = (int64_t)qi * f[0] + (int64_t)ri * g[0];
+        int64_t cd = (int64_t)ui * d[0] + (int64_t)vi * e[0];
+        int64_t ce = (int64_t)qi * d[0] + (int64_t)ri * e[0];
+        // P::INV = -1 / m mod 2^32: the multiples of m that clear the low 30 bits, in [-2^29, 2^29)
+        const int32_t md = (int32_t)((uint32_t)cd * P::INV << 2) >> 2;
+        const int32_t me = (int32_t)((uint32_t)ce * P::INV << 2) >> 2;
+        cd += (int64_t)md * modulus30<P>(0);
+        ce += (int64_t)me * modulus30<P>(0);
+        cf >>= 30;
+        cg >>= 30;
+        cd >>= 30;
+        ce >>= 30;
+#pragma unroll
+        for (int i = 1; i < 9; ++i) {
+            cf += (int64_t)ui * f[i] + (int64_t)vi * g[i];
+            cg += (int64_t)qi * f[i] + (int64_t)ri * g[i];
+            cd += (int64_t)ui * d[i] + (int64_t)vi * e[i] + (int64_t)md * modulus30<P>(i);
+            ce += (int64_t)qi * d[i] + (int64_t)ri * e[i] + (int64_t)me * modulus30<P>(i);
+            f[i - 1] = (int32_t)cf & M30;
+            g[i - 1] = (int32_t)cg & M30;
+            d[i - 1] = (int32_t)cd & M30;
+            e[i - 1] = (int32_t)ce & M30;
+            cf >>= 30;
+            cg >>= 30;
+            cd >>= 30;
+            ce >>= 30;
         }
-        for (int i = 0; i < 8; ++i)
-            o[i] = (r[i] >> 31) | (r[i + 1] << 1);
-        return neg;
-    };
-    // u, v update: (f p + g q + 2^32 m) / 2^32 mod m (one Montgomery step), p, q < m
-    auto modcomb = [&](const uint32_t (&p)[8], const uint32_t (&q)[8], int64_t f, int64_t g, uint32_t (&o)[8]) {
-        uint32_t r[9];
-        lincomb(p, q, f, g, r); // |r| <= 2^31 m
-        uint32_t t[10];
-        uint64_t c = 0; // + 2^32 m: nonnegative, below 2^33 m < 2^288
-        for (int i = 0; i < 10; ++i) {
-            const uint64_t rv = i < 9 ? (uint64_t)r[i] : ((int32_t)r[8] < 0 ? 0xffffffffull : 0ull);
-            const uint64_t mv = (i >= 1 && i <= 8) ? (uint64_t)P::M[i - 1] : 0ull;
-            const uint64_t s = rv + mv + c;
-            t[i] = (uint32_t)s;
-            c = s >> 32;
-        }
-        const uint32_t qm = t[0] * P::INV; // t + qm m = 0 mod 2^32
+        f[8] = (int32_t)cf; // the sign is the top limb's
+        g[8] = (int32_t)cg;
+        d[8] = (int32_t)cd;
+        e[8] = (int32_t)ce;
+    }
+    // d <- d * f (f = +-1), then into [0, m): |d| < 14 m
+    const bool neg = f[8] < 0;
+    int32_t c = 0;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        const int32_t t = (neg ? -d[i] : d[i]) + c;
+        d[i] = i < 8 ? t & M30 : t;
+        c = t >> 30;
+    }
+    for (int k = 0; k < 14 && d[8] < 0; ++k) {
         c = 0;
-        for (int i = 0; i < 10; ++i) {
-            const uint64_t s = (uint64_t)t[i] + (i < 8 ? (uint64_t)qm * P::M[i] : 0ull) + c;
-            t[i] = (uint32_t)s;
-            c = s >> 32;
-        }
-        for (int i = 0; i < 8; ++i) // (t + qm m) / 2^32 < 3m
-            o[i] = t[i + 1];
-        for (int k = 0; k < 2; ++k) {
-            uint32_t d[8];
-            int64_t bw = 0;
-            for (int i = 0; i < 8; ++i) {
-                const int64_t s = (int64_t)o[i] - (int64_t)P::M[i] + bw;
-                d[i] = (uint32_t)s;
-                bw = s >> 32;
-            }
-            if (bw == 0)
-                for (int i = 0; i < 8; ++i)
-                    o[i] = d[i];
-        }
-    };
-    for (int round = 0; round < 17; ++round) {
-        int n = bitlen(a) > bitlen(b) ? bitlen(a) : bitlen(b);
-        if (n < 64)
-            n = 64;
-        uint64_t at = ((uint64_t)a[0] & 0x7fffffffu) | (top33(a, n - 33) << 31);
-        uint64_t bt = ((uint64_t)b[0] & 0x7fffffffu) | (top33(b, n - 33) << 31);
-        int64_t f0 = 1, g0 = 0, f1 = 0, g1 = 1;
-        for (int j = 0; j < 31; ++j) {
-            if (at & 1) {
-                if (at < bt) {
-                    const uint64_t t = at;
-                    at = bt;
-                    bt = t;
-                    int64_t s = f0;
-                    f0 = f1;
-                    f1 = s;
-                    s = g0;
-                    g0 = g1;
-                    g1 = s;
-                }
-                at -= bt;
-                f0 -= f1;
-                g0 -= g1;
-            }
-            at >>= 1;
-            f1 *= 2;
-            g1 *= 2;
-        }
-        uint32_t ra[9], rb[9], na[8], nb[8];
-        lincomb(a, b, f0, g0, ra);
-        lincomb(a, b, f1, g1, rb);
-        if (shift31(ra, na)) {
-            f0 = -f0;
-            g0 = -g0;
-        }
-        if (shift31(rb, nb)) {
-            f1 = -f1;
-            g1 = -g1;
-        }
-        uint32_t nu[8], nv[8];
-        modcomb(u, v, f0, g0, nu);
-        modcomb(u, v, f1, g1, nv);
-        for (int i = 0; i < 8; ++i) {
-            a[i] = na[i];
-            b[i] = nb[i];
-            u[i] = nu[i];
-            v[i] = nv[i];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) {
+            const int32_t t = d[i] + modulus30<P>(i) + c;
+            d[i] = i < 8 ? t & M30 : t;
+            c = t >> 30;
         }
     }
-    // b = 1 = v x 2^(544 - 527): x^-1 = v 2^17 mod m
-    for (int k = 0; k < 17; ++k) {
-        uint32_t d[8];
-        uint32_t c = 0;
-        for (int i = 0; i < 8; ++i) { // v < m < 2^254: 2v < 2^255, no carry out
-            d[i] = (v[i] << 1) | c;
-            c = v[i] >> 31;
+    for (int k = 0; k < 14; ++k) {
+        int32_t s[9];
+        c = 0;
+#pragma unroll
+        for (int i = 0; i < 9; ++i) {
+            const int32_t t = d[i] - modulus30<P>(i) + c;
+            s[i] = i < 8 ? t & M30 : t;
+            c = t >> 30;
         }
-        uint32_t e[8];
-        int64_t bw = 0;
-        for (int i = 0; i < 8; ++i) {
-            const int64_t s = (int64_t)d[i] - (int64_t)P::M[i] + bw;
-            e[i] = (uint32_t)s;
-            bw = s >> 32;
-        }
-        for (int i = 0; i < 8; ++i)
-            v[i] = bw == 0 ? e[i] : d[i];
+        if (s[8] < 0)
+            break;
+#pragma unroll
+        for (int i = 0; i < 9; ++i)
+            d[i] = s[i];
     }
-    for (int i = 0; i < 8; ++i)
-        out[i] = v[i];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int q = 32 * i / 30, s = 32 * i % 30;
+        const uint64_t w = (uint64_t)(uint32_t)d[q] | (uint64_t)(uint32_t)d[q + 1] << 30;
+        out[i] = (uint32_t)(w >> s);
+    }
 }
 
 template <class P>
@@ -403,7 +394,7 @@ struct Fp256 {
         return r;
     }
 
-    // a^-1 by the binary extended GCD (inv_mod_plain): plain inverse of the
+    // a^-1 by division steps (inv_mod_plain): plain inverse of the
     // stored word A = a R, times R^3 with one Montgomery product (A^-1 R^2 = a^-1 R);
     // inverse_vt(0) = 0
     __device__ static Fp256 inverse_vt(const Fp256& a)

@@ -412,9 +412,9 @@ struct F29 {
     }
 
     // The same value as pow_m_minus_2 (u^-1 * 2^261 for a = u * 2^261, i.e.
-    // 2^522 / A for the integer A = a mod m; zero maps to zero) by the binary
-    // extended GCD (inv_mod_plain) and one product with 2^783. Input normalised,
-    // < 2m; output a normalised representative < 1.01m.
+    // 2^522 / A for the integer A = a mod m; zero maps to zero) by
+    // division steps (inv_mod_plain) and one product with 2^783, called by one lane of a
+    // wave only. Input normalised, < 2m; output a normalised representative < 1.01m.
     __device__ static F29 inverse_vt(const F29 a)
     {
         const F29 c = reduce_full(a);
@@ -422,7 +422,7 @@ struct F29 {
             return zero();
         uint32_t w[8], rw[8];
         c.to32(w);
-        inv_mod_plain<typename P::Base>(w, rw);
+        inv_mod_plain<typename P::Base, true>(w, rw);
         return mul(from32(rw), from_limbs(P::C783));
     }
 

@@ -1,4 +1,4 @@
-"""The scalar modular inversion (field.h inv_mod_plain, Pornin's batched binary GCD),
+"""The scalar modular inversion (field.h inv_mod_plain, batched division steps),
 built for the host from the same source and checked against Python's pow(x, -1, m) for
 both BN254 moduli: edge values (1, 2, m - 1, powers of two around the 64-bit
 approximation's boundaries, values just below m) and random ones of every length."""
