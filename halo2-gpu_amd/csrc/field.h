@@ -86,7 +86,7 @@ __host__ __device__ constexpr int32_t modulus30(int i)
 // their branches are scalar ones. What bounds that use is the chain of one lane: ~5 scalar
 // instructions a step in the rounds and ~90 multiply-adds after each. Against 31 plain steps of
 // the binary gcd on 64-bit images a round, the inversion of 128 totals (products.hip) takes
-// 77 us instead of 127.
+// 67 us instead of 127.
 template <class P, bool ONE = false>
 __host__ __device__ inline void inv_mod_plain(const uint32_t (&x)[8], uint32_t (&out)[8])
 {
@@ -107,6 +107,12 @@ __host__ __device__ inline void inv_mod_plain(const uint32_t (&x)[8], uint32_t (
         g[i] = (int32_t)((w >> s) & M30);
         d[i] = 0;
         e[i] = i == 0 ? 1 : 0;
+#ifdef __HIP_DEVICE_COMPILE__
+        if constexpr (ONE) { // in vector registers: v_mad_i64_i32 is one instruction, scalar four
+            asm("" : "+v"(f[i]), "+v"(g[i]));
+            asm("" : "+v"(d[i]), "+v"(e[i]));
+        }
+#endif
     }
     int theta = 0;
     for (int round = 0; round < 25; ++round) {
@@ -141,8 +147,12 @@ __host__ __device__ inline void inv_mod_plain(const uint32_t (&x)[8], uint32_t (
                 r = 0u - t;
                 theta = -theta - 1;
             }
-            int k = -theta < left ? -theta : left;
-            k = k < 6 ? k : 6;
+            int k = left < 6 ? left : 6;
+#ifdef __HIP_DEVICE_COMPILE__
+            if constexpr (ONE)
+                asm("" : "+s"(k)); // not a three-way minimum, which only the vector unit has
+#endif
+            k = -theta < k ? -theta : k;
             // f (2 - f^2) = 1 / f mod 2^6 (f is its own inverse mod 2^3)
             const uint32_t w = (gl * fl * (fl * fl - 2u)) & ((1u << k) - 1u);
             gl += fl * w;
