@@ -8,8 +8,8 @@
 // (FIPS, Koc-Acar-Kaliski 1996): every 32x32 partial product goes through one
 // `v_mad_u64_u32` into a 64-bit column accumulator whose carry-out feeds a
 // third accumulator word through `v_addc_co_u32`. This keeps the integer
-// multiply-add unit (64 lanes/clk/CU on gfx950) the only hot resource; no MFMA
-// because the arithmetic is exact modular integer work.
+// multiply-add unit (64 lanes/clk/CU on gfx950) the only hot resource.
+// (Products by the constants of a DFT run on the matrix cores: ntt_mfma.h.)
 //
 // Constants (moduli, -m^-1 mod 2^32, R mod m, R^2 mod m) are BN254's; the
 // reference keeps the same values at cuda/include/field/alt_bn128.hpp:19-47.

@@ -494,7 +494,8 @@ RustError h2amd_msm_set_widths(const uint8_t* widths, uint32_t count);
 uint32_t h2amd_msm_width(uint64_t n);
 uint32_t h2amd_msm_table_width(uint64_t table_n);
 /* tiles[log_n] (0 = default, else 6..12): log2 of the elements one NTT work-group
- * transforms (radix columns x column group) for transforms of 2^log_n; same rules. */
+ * transforms (radix columns x column group) for transforms of 2^log_n; same rules. A pass
+ * takes at least 2^9, so 6..8 act as 9. */
 RustError h2amd_ntt_set_tiles(const uint8_t* tiles, uint32_t count);
 
 /* ======================= kernel timing (no reference counterpart)
