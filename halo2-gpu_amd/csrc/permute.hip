@@ -317,27 +317,15 @@ __device__ __forceinline__ TileSpan tile_span(uint64_t tile, uint64_t U, uint64_
     return t;
 }
 
-// Merge-path splits of one merge pass: for each key array y, output tile and
-// end (0 = first output, 1 = one past the last), the number of keys the tile
-// takes from run A, at splits[(y * tiles + tile) * 2 + end]. One wave per
-// split narrows the range with 64 probes per round (a 64-ary search), so a
-// run of 2^21 keys takes four rounds of dependent loads instead of 21.
-__global__ void __launch_bounds__(256) run_split_kernel(const Key* __restrict__ keys, uint64_t* __restrict__ splits,
-    uint64_t U, uint64_t stride, uint64_t w, uint32_t tiles)
+// Merge-path split: the number of keys that the first d outputs of a pair of runs take from run
+// A. The wave narrows the range with 64 probes per round (a 64-ary search), so a run of 2^21
+// keys takes four rounds of dependent loads instead of 21.
+__device__ __forceinline__ uint64_t wave_split(const Key* A, const Key* B, uint64_t na, uint64_t nb, uint64_t d,
+    uint32_t lane)
 {
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const uint32_t lane = threadIdx.x & 63u;
-    if (wave >= tiles * 4u) // uniform per wave
-        return;
-    const uint32_t y = wave / (tiles * 2u);
-    const uint32_t rem = wave % (tiles * 2u);
-    const TileSpan t = tile_span(rem >> 1, U, w);
-    const uint64_t d = (rem & 1u) ? t.d1 : t.d0;
-    const Key* A = keys + y * stride + t.pair;
-    const Key* B = A + t.na;
     // first i in [lo, hi) with B[d - 1 - i] < A[i] (ties go to A), else hi
-    uint64_t lo = d > t.nb ? d - t.nb : 0;
-    uint64_t hi = d < t.na ? d : t.na;
+    uint64_t lo = d > nb ? d - nb : 0;
+    uint64_t hi = d < na ? d : na;
     while (lo < hi) {
         const uint64_t step = (hi - lo + 63) >> 6;
         const uint64_t i = lo + lane * step;
@@ -352,18 +340,18 @@ __global__ void __launch_bounds__(256) run_split_kernel(const Key* __restrict__ 
                 hi = first_false;
         }
     }
-    if (lane == 0)
-        splits[wave] = lo;
+    return lo;
 }
 
 // One merge pass: runs of length w (sorted) merged pairwise into runs of 2w,
-// 2048 outputs per work-group of 1024 threads (two each) between the splits
-// run_split_kernel found.
+// 2048 outputs per work-group of 1024 threads (two each). Two waves find the tile's splits
+// while the other work-group of the compute unit loads or merges: a launch of its own for
+// the splits took 8 us a pass beside 31 for the merge at 2^20 keys, the two together take 36.
 constexpr unsigned kMergeThreads = 1024;
 constexpr unsigned kMergePer = kTile / kMergeThreads;
 
 __global__ void __launch_bounds__(kMergeThreads) merge_pass_kernel(const Key* __restrict__ keys,
-    Key* __restrict__ out, const uint64_t* __restrict__ splits, uint64_t U, uint64_t stride, uint64_t w)
+    Key* __restrict__ out, uint64_t U, uint64_t stride, uint64_t w)
 {
     __shared__ Key sh[kTile];
     const Key* src = keys + blockIdx.y * stride;
@@ -371,7 +359,13 @@ __global__ void __launch_bounds__(kMergeThreads) merge_pass_kernel(const Key* __
     const TileSpan ts = tile_span(blockIdx.x, U, w);
     const Key* A = src + ts.pair;
     const Key* B = A + ts.na;
-    const uint64_t* sp = splits + ((uint64_t)blockIdx.y * gridDim.x + blockIdx.x) * 2;
+    __shared__ uint64_t sp[2];
+    if (threadIdx.x < 128) { // wave 0: first output, wave 1: one past the last
+        const uint64_t i = wave_split(A, B, ts.na, ts.nb, threadIdx.x < 64 ? ts.d0 : ts.d1, threadIdx.x & 63u);
+        if ((threadIdx.x & 63u) == 0)
+            sp[threadIdx.x >> 6] = i;
+    }
+    __syncthreads();
     const uint64_t a0 = sp[0], a1 = sp[1];
     const uint64_t b0 = ts.d0 - a0, b1 = ts.d1 - a1;
     const uint32_t ta = (uint32_t)(a1 - a0), tb = (uint32_t)(b1 - b0);
@@ -474,7 +468,6 @@ struct PermBufs {
     uint32_t* leftover;
     uint32_t* rpos;
     uint32_t* lpos;
-    uint64_t* splits; // merge-path splits of one pass: 2 arrays x tiles x 2
     void* scan;
 };
 
@@ -488,7 +481,6 @@ PermBufs perm_carve(WS& ws, uint64_t U)
     b.leftover = (uint32_t*)ws.take(4 * U);
     b.rpos = (uint32_t*)ws.take(4 * (U + 1));
     b.lpos = (uint32_t*)ws.take(4 * (U + 1));
-    b.splits = (uint64_t*)ws.take(8 * 4 * ((U + kTile - 1) / kTile));
     b.scan = ws.take(scan_u32_scratch(U));
     return b;
 }
@@ -546,11 +538,7 @@ RustError _halo2_permute_expression_pair(const void* d_compressed_input, const v
         H2_LAUNCH_CHECK();
         int cur = 1;
         for (uint64_t w = kSortTile; w < U; w <<= 1) {
-            run_split_kernel<<<blocks_for(4ull * tiles * 64, 256), 256, 0, stream>>>(b.keys[cur], b.splits, U, U, w,
-                tiles);
-            H2_LAUNCH_CHECK();
-            merge_pass_kernel<<<dim3(tiles, 2), kMergeThreads, 0, stream>>>(b.keys[cur], b.keys[cur ^ 1], b.splits, U, U,
-                w);
+            merge_pass_kernel<<<dim3(tiles, 2), kMergeThreads, 0, stream>>>(b.keys[cur], b.keys[cur ^ 1], U, U, w);
             H2_LAUNCH_CHECK();
             cur ^= 1;
         }
