@@ -22,7 +22,10 @@ _MONT_INV = {R_MOD: pow(MONT, -1, R_MOD), P_MOD: pow(MONT, -1, P_MOD)}
 
 
 def limbs(x: int) -> np.ndarray:
-    return np.frombuffer(bytearray((x & (MONT - 1)).to_bytes(32, "little")), dtype=np.uint64)
+    if isinstance(x, int):
+        return np.frombuffer(bytearray((x & (MONT - 1)).to_bytes(32, "little")), dtype=np.uint64)
+    # numpy's unsigned 64-bit integers, which take no mask of 256 bits
+    return np.array([(x >> (64 * i)) & 0xFFFFFFFFFFFFFFFF for i in range(4)], dtype=np.uint64)
 
 
 def from_limbs(a) -> int:
