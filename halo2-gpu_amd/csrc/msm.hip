@@ -180,13 +180,18 @@ uint32_t plain_msm_width(uint64_t npoints)
     return default_width(2 * npoints, false, GLV_BITS);
 }
 
+constexpr uint32_t kR1Groups = 512; // round-1 work-groups wanted
+// an MSM with less work than kShortRunThreads threads of kShortRun entries each runs in such threads
+constexpr uint64_t kShortRun = 8;
+constexpr uint64_t kShortRunThreads = 1ull << 16;
+
 // Few tiles leave compute units idle while each tile goes through its windows one after the
 // other (~4 us each), so a tile's windows are dealt to several work-groups, up to ~2 per compute
 // unit: round 1 of a 1500 point MSM 137 -> 37 us, of 50 003 points 109 -> 46.
 void set_tiles(MsmPlan& p, uint32_t ntiles)
 {
     p.ntiles = ntiles;
-    uint32_t groups = ntiles ? 512 / ntiles : 1;
+    uint32_t groups = ntiles ? kR1Groups / ntiles : 1;
     groups = groups < 1 ? 1 : groups > p.W ? p.W : groups;
     p.wper = (p.W + groups - 1) / groups;
     p.groups = (p.W + p.wper - 1) / p.wper;
@@ -225,7 +230,7 @@ MsmPlan plan_core(uint64_t n, uint32_t c, uint32_t J, uint64_t table_n, uint32_t
     // one thread's chain (1500 points 365 -> 341 us, three 2^12 table MSMs 377 -> 338;
     // five of 2^16 would go from 0.89 to 0.99 ms)
     uint64_t s = work >> 20;
-    const uint64_t least = work < (8ull << 16) ? 8 : 16;
+    const uint64_t least = work < kShortRun * kShortRunThreads ? kShortRun : 16;
     if (s < least)
         s = least;
     if (s > 128)
@@ -272,17 +277,8 @@ MsmPlan make_plan(uint64_t n, uint64_t table_n = 0)
 
 uint64_t align_tile(uint64_t n) { return (n + R1_TILE - 1) / R1_TILE * R1_TILE; }
 
-// J MSMs over one shared base array (or one precomputed table of table_n
-// points): one width for all (from the mean job size, or the table's), each
-// job's points at a tile-aligned virtual offset.
-MsmPlan make_batch_plan(const uint64_t* lengths, uint32_t J, uint64_t table_n = 0)
+MsmPlan batch_plan(uint64_t nv, uint64_t nmax, uint32_t J, uint64_t table_n)
 {
-    uint64_t nv = 0, nmax = 0;
-    for (uint32_t j = 0; j < J; ++j) {
-        nv += align_tile(lengths[j]);
-        if (lengths[j] > nmax)
-            nmax = lengths[j];
-    }
     const uint64_t mean = nv / J ? nv / J : 1;
     uint32_t c = table_n ? plan_width(table_n, true) : plan_width(mean, false);
     if (!table_n && c > 16) // J * W * 2^(c-1) buckets of 128 B: 4 GiB at most for 64 jobs
@@ -294,6 +290,20 @@ MsmPlan make_batch_plan(const uint64_t* lengths, uint32_t J, uint64_t table_n = 
     p.pts_count = nmax;
     p.batch = true;
     return p;
+}
+
+// J MSMs over one shared base array (or one precomputed table of table_n
+// points): one width for all (from the mean job size, or the table's), each
+// job's points at a tile-aligned virtual offset.
+MsmPlan make_batch_plan(const uint64_t* lengths, uint32_t J, uint64_t table_n = 0)
+{
+    uint64_t nv = 0, nmax = 0;
+    for (uint32_t j = 0; j < J; ++j) {
+        nv += align_tile(lengths[j]);
+        if (lengths[j] > nmax)
+            nmax = lengths[j];
+    }
+    return batch_plan(nv, nmax, J, table_n);
 }
 
 struct MsmBuffers {
@@ -322,10 +332,26 @@ struct MsmBuffers {
 // bins (a table), each of its work-groups does
 uint64_t r1_counts(const MsmPlan& p) { return (uint64_t)p.NCj * p.ntiles * (p.table_n ? p.groups : 1); }
 
+// What the buffers of round-1 counters and of partial sums are sized for: as much as any MSM of
+// fewer points takes at this width, so that one scratch serves every length up to the one that
+// it was sized for (fewer points have more work-groups per tile and shorter runs per thread)
+uint64_t r1_counts_room(const MsmPlan& p)
+{
+    const uint64_t most = kR1Groups < (uint64_t)p.ntiles * p.W ? kR1Groups : (uint64_t)p.ntiles * p.W;
+    return p.NCj * (p.table_n && most > p.ntiles ? most : p.ntiles);
+}
+
+uint64_t part_room(const MsmPlan& p)
+{
+    const uint64_t short_runs = (p.n * p.W + kShortRun - 1) / kShortRun;
+    const uint64_t most = short_runs < kShortRunThreads ? short_runs : kShortRunThreads;
+    return p.nthr > most ? p.nthr : most;
+}
+
 template <class WS>
 void carve(WS& ws, const MsmPlan& p, MsmBuffers* b)
 {
-    const uint64_t nh1 = r1_counts(p);
+    const uint64_t nh1 = r1_counts_room(p);
     const uint64_t nh2 = p.max_chunks << p.FB;
     uint64_t scan_n = nh1 + 1;
     if (nh2 + 1 > scan_n)
@@ -352,7 +378,7 @@ void carve(WS& ws, const MsmPlan& p, MsmBuffers* b)
     v[k++] = ws.take(4 * p.n * p.W);
     v[k++] = ws.take(4 * (p.nb + 1));
     v[k++] = ws.take(4 * (p.nb + 1));
-    v[k++] = ws.take(128 * 2 * p.nthr);
+    v[k++] = ws.take(128 * 2 * part_room(p));
     v[k++] = ws.take(128 * p.nb);
     for (int i = 0; i < 2; ++i)
         v[k++] = ws.take(128 * nred[i]);
@@ -392,12 +418,25 @@ struct SizerAdapter {
     }
 };
 
-uint64_t msm_workspace_bytes(uint64_t n, uint64_t table_n = 0)
+uint64_t plan_bytes(const MsmPlan& p)
 {
-    MsmPlan p = make_plan(n, table_n);
     SizerAdapter sa;
     carve(sa, p, nullptr);
     return sa.s.bytes + 4096;
+}
+
+// Scratch for n points. Without a table the width follows n, and fewer points at a narrower
+// width can take more (more windows), so it is the most that n points or the last length below
+// each power of two up to 2^18 take. (From 2^19 points on a scratch serves the length it was
+// sized for only.)
+uint64_t msm_workspace_bytes(uint64_t n, uint64_t table_n = 0)
+{
+    uint64_t most = plan_bytes(make_plan(n, table_n));
+    for (uint32_t k = 1; !table_n && k <= 18 && (1ull << k) <= n; ++k) {
+        const uint64_t bytes = plan_bytes(make_plan((1ull << k) - 1));
+        most = bytes > most ? bytes : most;
+    }
+    return most;
 }
 
 // ------------------------------------------------------------- kernels
@@ -1791,7 +1830,7 @@ RustError _halo2_multiexp_device_scalars_device_bases(const void* d_scalar, cons
 namespace {
 
 constexpr uint64_t kNoAllocMaxLength = 1ull << 16;
-constexpr uint64_t kNoAllocScratchBytes = 64ull << 20; // >= msm_workspace_bytes(2^16) at default widths
+constexpr uint64_t kNoAllocScratchBytes = 64ull << 20; // >= what 2^16 points take at default widths
 
 __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 
@@ -1830,7 +1869,7 @@ RustError h2amd_multiexp_device_scalars_device_bases_noalloc(const void* d_scala
     const char* who = "h2amd_multiexp_device_scalars_device_bases_noalloc";
     H2_CHECK_ARG(length <= kNoAllocMaxLength, "%s: length %lu exceeds the built-in scratch's maximum of %lu points",
         who, (unsigned long)length, (unsigned long)kNoAllocMaxLength);
-    const uint64_t need = msm_workspace_bytes(length);
+    const uint64_t need = plan_bytes(make_plan(length));
     H2_CHECK_ARG(need <= kNoAllocScratchBytes,
         "%s: length %lu needs %lu bytes of scratch at the current window width, the built-in scratch holds %lu", who,
         (unsigned long)length, (unsigned long)need, (unsigned long)kNoAllocScratchBytes);
@@ -1923,10 +1962,15 @@ uint64_t h2amd_multiexp_batch_workspace_size(const uint64_t* lengths, uint32_t c
 {
     if (count == 0 || count > MAX_JOBS)
         return 0;
+    // as msm_workspace_bytes: the width follows the mean length
     const MsmPlan p = make_batch_plan(lengths, count);
-    SizerAdapter sa;
-    carve(sa, p, nullptr);
-    return sa.s.bytes + 4096;
+    uint64_t most = plan_bytes(p);
+    for (uint32_t k = 1; k <= 20 && ((uint64_t)count << k) <= p.n; ++k) {
+        const uint64_t nv = (((uint64_t)count << k) - 1) / R1_TILE * R1_TILE;
+        const uint64_t bytes = plan_bytes(batch_plan(nv, p.nbase, count, 0));
+        most = bytes > most ? bytes : most;
+    }
+    return most;
 }
 
 // J MSMs in one pipeline over shared bases (table_n = 0) or one precomputed table
@@ -1993,10 +2037,7 @@ uint64_t h2amd_multiexp_batch_precomputed_workspace_size(const uint64_t* lengths
 {
     if (count == 0 || count > MAX_JOBS || table_n == 0)
         return 0;
-    const MsmPlan p = make_batch_plan(lengths, count, table_n);
-    SizerAdapter sa;
-    carve(sa, p, nullptr);
-    return sa.s.bytes + 4096;
+    return plan_bytes(make_batch_plan(lengths, count, table_n));
 }
 
 RustError h2amd_multiexp_batch_precomputed(const void* const* d_scalars, const uint64_t* lengths, uint32_t count,

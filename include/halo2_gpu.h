@@ -419,6 +419,9 @@ uint64_t h2amd_msm_precompute_workspace_size(uint64_t n);
 /* d_table (h2amd_msm_table_bytes(n) bytes) from n device affine bases */
 RustError h2amd_msm_precompute(void* d_table, const void* d_bases, uint64_t n, void* scratch,
     uint64_t scratch_bytes, void* stream);
+/* As every MSM scratch here, one sized for `length` also serves fewer points (over the same
+ * table, under the same widths) while an MSM has fewer than 2^24 digits (length x windows);
+ * without a table, up to 2^19 - 1 points. Above, it serves the length that it was sized for. */
 uint64_t h2amd_multiexp_precomputed_workspace_size(uint64_t length, uint64_t table_n);
 /* sum_i s_i P_i over the first `length` <= table_n points of a table built for table_n
  * points; device scalars, host 96-byte output (as `_halo2_multiexp_*`). Synchronises. */

@@ -557,3 +557,21 @@ def test_msm_batch_of_one(lib, co, n):
         torch.cuda.synchronize()
         del stale
         assert (msm.multiexp_batch_precomputed([d_c], table, n)[0] == exp).all()
+
+
+@pytest.mark.parametrize("n", [1, 4097, 30784, (1 << 15) - 1])
+def test_msm_table_scratch_of_the_whole_length(lib, co, n):
+    """One scratch, sized for a table's whole length, for shorter polynomials."""
+    import ctypes
+
+    from halo2_amd import _lib, device as dv, msm
+
+    m = 1 << 15
+    pts, c = co.g1_mul_gen(rand_fr(co, m, 41)), rand_fr(co, n, 42 + n)
+    table = msm.msm_precompute(dv.to_device(pts), m)
+    ws = int(lib.h2amd_multiexp_precomputed_workspace_size(m, m))
+    scratch, d_c, out = dv.empty_bytes(ws), dv.to_device(c), np.zeros(12, dtype=np.uint64)
+    obj = _lib.obj(out.ctypes.data)
+    _lib.check(lib.h2amd_multiexp_precomputed(dv.ptr(d_c), dv.ptr(table), m, ctypes.byref(obj), n, dv.ptr(scratch), ws,
+                                              dv.stream()), "h2amd_multiexp_precomputed")
+    assert (out == co.msm(c, pts[:n])).all()
