@@ -820,10 +820,17 @@ static hipError_t raise_lds_limits()
     return status;
 }
 
-// Threads per work-group: 8 waves where a tile has work for them (a unit of a matrix step is
-// 512 elements) or where the launch leaves compute units idle anyway; 4 otherwise, so two
-// work-groups share a compute unit and one's memory phases overlap the other's products.
-static uint32_t pass_threads(uint32_t rg, uint64_t groups) { return rg >= 4096 || groups < 256 ? 512 : 256; }
+// Threads per work-group: 8 waves where a compute unit gets one work-group (its tile takes more
+// than half of the LDS, or there are no more work-groups than compute units) or a tile has work
+// for them (a unit of a matrix step is 512 elements); 4 otherwise, so that two work-groups share a
+// compute unit and one's memory phases overlap the other's products. With 4 waves for 256
+// work-groups and for tiles of 2048 in 84 KiB a single 2^19 took 111 us, now 97, eight of them
+// 594, now 518 (2^18: 72, 66; 2^17: 52.2, 49.7); with 8 waves everywhere eight of 2^17 take 213
+// instead of 161.
+static uint32_t pass_threads(uint32_t rg, uint64_t groups, uint32_t lds_bytes)
+{
+    return rg >= 4096 || groups <= 256 || 2 * lds_bytes > kMaxPassLds ? 512 : 256;
+}
 
 RustError ntt_run(const NttTables& t, uint32_t log_n, const NttJob* jobs, int count, uint64_t in_len,
     Fr* scratch, uint64_t scratch_slots, NttTwist twist, NttPost post, const Fr& scale, hipStream_t stream)
@@ -900,8 +907,8 @@ RustError ntt_run(const NttTables& t, uint32_t log_n, const NttJob* jobs, int co
             dim3 grid(nwg, nb);
             {
                 ProfScope prof("ntt_pass", stream);
-                ntt_pass_kernel<<<grid, pass_threads(RG, (uint64_t)nwg * nb), pass_lds_bytes(pp.log_r, pp.log_g, pp.last),
-                    stream>>>(pb, pp);
+                const uint32_t lds = pass_lds_bytes(pp.log_r, pp.log_g, pp.last);
+                ntt_pass_kernel<<<grid, pass_threads(RG, (uint64_t)nwg * nb, lds), lds, stream>>>(pb, pp);
             }
             H2_LAUNCH_CHECK();
         }
@@ -997,7 +1004,7 @@ RustError ntt_run_batch(const NttBatchJob* jobs, int count, NttTwist twist, NttP
         if (!nlaunch[pass])
             continue;
         ProfScope prof("ntt_pass_batch", stream);
-        ntt_pass_batch_kernel<<<grid[pass], pass_threads(1u << rgmax[pass], grid[pass]), lds[pass],
+        ntt_pass_batch_kernel<<<grid[pass], pass_threads(1u << rgmax[pass], grid[pass], lds[pass]), lds[pass],
             stream>>>(dp + (uint64_t)pass * count, nlaunch[pass]);
         H2_LAUNCH_CHECK();
     }
