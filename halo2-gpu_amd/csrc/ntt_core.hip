@@ -128,18 +128,21 @@ static std::atomic<uint8_t> g_tile_table[NTT_MAX_LOG + 1] = {};
 NttPlan ntt_plan(uint32_t log_n)
 {
     NttPlan p {};
-    if (log_n <= NTT_MAX_LOG_R) {
-        p.P = 1;
-        p.log_r[0] = log_n;
-    } else if (log_n <= 2 * NTT_MAX_LOG_R) {
-        p.P = 2;
+    p.P = log_n <= NTT_MAX_LOG_R ? 1 : log_n <= 2 * NTT_MAX_LOG_R ? 2 : 3;
+    // A pass of 2^8 rows takes two matrix steps (16 x 16), one of 2^9 to 2^12 three: where the first
+    // pass can hold the rest, all later ones are of 2^8 (2^17 .. 2^20: 5 steps; 2^25 .. 2^28: 7).
+    // Even splits take 6 and up to 9: 2^20 153 -> 147 us, 2^27 24.5 -> 23.5 ms, twelve of 2^18 in an
+    // uneven batch 380 -> 349 us. Else (2^13 .. 2^16: 4 steps, 2^21 .. 2^24: 6) passes are about even.
+    const uint32_t rest = log_n > 8u * (p.P - 1) ? log_n - 8u * (p.P - 1) : 0;
+    if (p.P > 1 && rest >= 9 && rest <= NTT_MAX_LOG_R) {
+        p.log_r[0] = rest;
+        for (int i = 1; i < p.P; ++i)
+            p.log_r[i] = 8;
+    } else if (p.P == 2) {
         p.log_r[0] = (log_n + 1) / 2;
         p.log_r[1] = log_n - p.log_r[0];
     } else {
-        p.P = 3;
-        p.log_r[0] = (log_n + 2) / 3;
-        p.log_r[1] = (log_n - p.log_r[0] + 1) / 2;
-        p.log_r[2] = log_n - p.log_r[0] - p.log_r[1];
+        p.log_r[0] = log_n;
     }
     for (int i = 0; i < p.P; ++i) {
         // aim for >= 256 work-groups per transform, 512 to 4096 elements per work-group (a
@@ -980,9 +983,10 @@ RustError ntt_run_batch(const NttBatchJob* jobs, int count, NttTwist twist, NttP
             pp.last_matrices = jb.tables->last_matrices;
             if (jb.log_n >= NTT_MATRIX_LOG)
                 pp.steps = radix_steps(pp.log_r);
-            pp.xcd_remap = 0;
             const uint32_t rg = pp.log_r + pp.log_g;
             bp.nwg = (uint32_t)((1ull << jb.log_n) >> (pp.log_r + pp.log_g));
+            // as ntt_run (two of 2^22 1046 -> 1001 us); the transform's first block only rotates the XCDs
+            pp.xcd_remap = (bp.nwg % 8 == 0 && bp.nwg >= 64) ? 1u : 0u;
             bp.block0 = grid[pass];
             grid[pass] += bp.nwg;
             if (rg > rgmax[pass])

@@ -438,3 +438,39 @@ def test_batch_of_every_small_size(lib, co, po, kind):
     outs = ntt.fft_batch_to_device(kind, [dv.to_device(a) for a in ins], ks, ks, omegas, divs)
     for k, a, o in zip(ks, ins, outs):
         assert (dv.to_host(o) == _oracle_kind(co, po, kind, a, k, c=c)).all(), k
+
+
+@pytest.mark.parametrize("kind", [1, 6])
+def test_batch_of_middle_sizes(lib, co, po, kind):
+    """One uneven batch of 2^16 .. 2^20, whose passes are split in different ways."""
+    from halo2_amd import device as dv, fields as F, ntt
+
+    ks = [17, 20, 18, 16, 19, 18]
+    ins = [rand_fr(co, 1 << k, 970 + i) for i, k in enumerate(ks)]
+    c = 0xABCDEF987654321
+    outs = ntt.fft_batch_to_device(kind, [dv.to_device(a) for a in ins], ks, ks, [F.omega(k) for k in ks], [c] * len(ks))
+    for k, a, o in zip(ks, ins, outs):
+        assert (dv.to_host(o) == _oracle_kind(co, po, kind, a, k, c=c)).all(), k
+
+
+@pytest.mark.parametrize("k", [18, 20, 21, 25, 26, 27, 28])
+def test_large_transform_of_few_values(lib, k):
+    """a e_i + b e_j has the transform a w^(i m) + b w^(j m): every split of the passes of the
+    largest sizes, with another root than the default one, at 2000 places and both ends."""
+    import torch
+
+    from halo2_amd import device as dv, fields as F, ntt
+
+    n, w = 1 << k, pow(F.omega(k), 5, F.R_MOD)
+    rng = np.random.default_rng(k)
+    i, j = n - 1, int(rng.integers(1, n // 2)) | 1
+    a, b = 3, 0x1234567890ABCDEF << 180
+    d = torch.zeros(4 * n, dtype=torch.int64, device="cuda")
+    for at, v in ((i, a), (j, b)):
+        d[4 * at:4 * at + 4] = torch.from_numpy(F.mont_limbs(v).view(np.int64)).cuda()
+    out = dv.empty_u64(4 * n)
+    ntt.fft_normal_device(ntt.FFT, k, d, out, w, 1)
+    ms = np.unique(np.concatenate([[0, 1, n - 1, n // 2], rng.integers(0, n, 2000)]))
+    got = out.view(-1, 4)[torch.from_numpy(ms).cuda()].cpu().numpy().view(np.uint64)
+    for m, row in zip(ms.tolist(), got):
+        assert F.value_of(row) == (a * pow(w, i * m % n, F.R_MOD) + b * pow(w, j * m % n, F.R_MOD)) % F.R_MOD, m
