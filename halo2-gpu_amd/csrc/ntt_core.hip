@@ -646,12 +646,15 @@ __device__ __forceinline__ void pass_twiddles(const PassParams& pp, uint4* T, ui
 }
 
 // A transform of fewer points than a matrix step takes (2 to 32): y_k = sum_i x_i w^(ik) by
-// definition, one thread per output, at most 32 products deep.
+// definition. Eight threads per output take every eighth term, at most 4 products deep (one
+// thread per output was 32 deep: a call of 2^5 points 36 us, now 29, the host's part).
 __device__ __forceinline__ void ntt_direct(const Fr* __restrict__ in, Fr* __restrict__ out, const PassParams& pp,
     uint4* lds)
 {
-    const uint32_t N = 1u << pp.log_n, k = threadIdx.x;
-    if (k < N) {
+    constexpr uint32_t kParts = 8; // 8 N <= 256 threads
+    const uint32_t N = 1u << pp.log_n, k = threadIdx.x & (N - 1), part = threadIdx.x >> pp.log_n;
+    uint4* sums = lds + 2 * N;
+    if (part == 0) {
         Fr29 x = Fr29::zero();
         if (k < pp.in_len) {
             x = Fr29::load32(in + k);
@@ -661,16 +664,24 @@ __device__ __forceinline__ void ntt_direct(const Fr* __restrict__ in, Fr* __rest
         lds_store(lds, k, x);
     }
     __syncthreads();
-    if (k >= N)
+    if (part < kParts) {
+        Fr29 y = Fr29::zero();
+        for (uint32_t i = part; i < N; i += kParts) {
+            const uint4* p = lds + 2 * lds_slot(i);
+            // x < 5.3 m (2^256): each product < 1.04 m, the sum < 4.2 m < 2^256
+            y = Fr29::normalize(Fr29::add(y, Fr29::mul(Fr29::load32(p), Fr29::load32(pp.twr + ((i * k) & (N - 1))))));
+        }
+        lds_store(sums, part * N + k, y);
+    }
+    __syncthreads();
+    if (part)
         return;
     Fr29 y = Fr29::zero();
-    for (uint32_t i = 0; i < N; ++i) {
-        const uint4* p = lds + 2 * lds_slot(i);
-        // x < 5.3 m (2^256): each product < 1.04 m, the sum < 34 m
-        y = Fr29::normalize(Fr29::add(y, Fr29::mul(Fr29::load32(p), Fr29::load32(pp.twr + ((i * k) & (N - 1))))));
-    }
+#pragma unroll
+    for (uint32_t i = 0; i < kParts; ++i) // limbs < 8 2^29
+        y = Fr29::add(y, Fr29::load32(sums + 2 * lds_slot(i * N + k)));
     const Fr29 w = post_constant(pp, pp.post == POST_SCALE_ZETA_INV ? k % 3u : 0u);
-    canonical_3m(Fr29::mul(y, w)).store32(out + k); // < 1.25 m before
+    canonical_3m(Fr29::mul(Fr29::normalize(y), w)).store32(out + k); // < 1.25 m before
 }
 
 // Work-group `b` (of nwg) of one pass of one transform. Every value in LDS is < 2.1 m, or
