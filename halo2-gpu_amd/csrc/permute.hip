@@ -137,14 +137,26 @@ __device__ __forceinline__ void merge_run(const Key* A, uint32_t na, const Key* 
 //
 // What is sorted is not the 32-byte keys but 64-bit words of 51 key bits and the key's 13-bit
 // place in the tile, four times less to move through LDS and registers; the keys themselves
-// are read where they lie and written once, in order. The 51 bits are the window below the
-// highest bit in which the tile's keys differ. If no lower bit exists the words order the
-// keys completely; otherwise neighbours that agree in the window are compared, and only if
-// two of them differ (2^-26 a tile for uniform keys) the tile is sorted again by all its
-// windows, lowest first (the place in the current order keeps each round stable).
+// are read where they lie and written once, in order. Which 51 bits:
+//  - the tile's keys differ in 51 bits at most: those, and the order is complete;
+//  - otherwise the window below the highest bit in which they differ. It is checked: the keys of
+//    neighbours that agree in it are compared. For uniform keys it holds but for 2^-26 a tile;
+//  - if it does not hold, which a look at neighbouring keys mostly shows before the sort (signed
+//    small numbers: m - x and x share all the window), the bits that tell keys apart. The highest
+//    bit in which two keys differ, for every two neighbours of a sorted order, is enough to
+//    compare any two keys; neighbours of an unsorted order give most of these bits, and the ones
+//    right below them, as far as 51 reach, the rest. All neighbours' keys are then compared;
+//  - if there are too many such bits, the keys' lengths vary (powers of two, say): the length and
+//    the 43 bits below the highest one, checked in the same way;
+//  - after that, or two rounds of chosen bits, the tile is sorted by all the bits in which its keys
+//    differ, 51 a round and the lowest first (the place in the current order keeps each round stable).
 // Words are sorted 8 per thread in registers, then in ten merge rounds.
 // 2^20 rows of two columns: 213 us with keys as the words and 2048 a tile, now 85, and two
-// merge passes of 38 us less.
+// merge passes of 38 us less. The whole call for signed numbers, 2^10, 2^16 and 2^20 rows: 92,
+// 188, 713 us with keys as the words, now 75, 158, 603 (263, 360, 754 if a tile that ties in its
+// window goes through all of them); for powers of two 91, 183, 683 and now 74, 156, 510. Keys that
+// need all the bits (40 lengths with more than 43 bits below) take longer: 88, 175, 671 and 239,
+// 362, 772.
 constexpr unsigned kSortThreads = 1024;
 constexpr unsigned kSortPer = kSortTile / kSortThreads;
 constexpr unsigned kIndexBits = 13;
@@ -219,23 +231,140 @@ __device__ __forceinline__ void sort_words(uint64_t* sh)
     __syncthreads();
 }
 
+// A choice of at most 51 key bits as runs within the key's words, highest first:
+// word << 16 | lowest bit << 8 | bits
+struct BitRuns {
+    uint32_t count;
+    uint32_t run[kWindow];
+};
+
+__device__ inline void set_runs(BitRuns& runs, const uint64_t (&mask)[4])
+{
+    uint32_t n = 0;
+    for (int q = 3; q >= 0; --q) {
+        uint64_t m = mask[q];
+        while (m) {
+            const uint32_t top = 63 - __builtin_clzll(m);
+            const uint64_t holes = ~(m << (63 - top));
+            const uint32_t bits = holes ? __builtin_clzll(holes) : 64;
+            const uint32_t low = top + 1 - bits;
+            runs.run[n++] = (uint32_t)q << 16 | low << 8 | bits;
+            m &= (1ull << low) - 1;
+        }
+    }
+    runs.count = n;
+}
+
+// m |= m >> n, 0 < n < 64
+__device__ __forceinline__ void or_shifted(uint64_t (&m)[4], uint32_t n)
+{
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+        m[q] |= m[q] >> n | m[q + 1] << (64 - n);
+    m[3] |= m[3] >> n;
+}
+
+__device__ __forceinline__ uint32_t bits_set(const uint64_t (&m)[4])
+{
+    return __popcll(m[0]) + __popcll(m[1]) + __popcll(m[2]) + __popcll(m[3]);
+}
+
+// a place 1 to 8 after k, by turns of no regular period (columns often interleave a few sequences)
+__device__ __forceinline__ uint32_t near_to(uint32_t k, uint32_t count)
+{
+    const uint32_t other = k + 1 + ((k * 0x9e3779b1u) >> 29);
+    return other < count ? other : count - 1;
+}
+
+// the words of the tile's keys (in the order `perm`, if any) by a choice of bits
+__device__ __forceinline__ void words_by_runs(uint64_t* sh, const Key* __restrict__ src, uint32_t count,
+    const BitRuns& runs, const uint16_t* perm = nullptr)
+{
+    uint64_t v[kSortPer];
+    uint32_t from[kSortPer];
+#pragma unroll
+    for (unsigned k = 0; k < kSortPer; ++k) {
+        v[k] = 0;
+        from[k] = perm ? perm[threadIdx.x + k * kSortThreads] : threadIdx.x + k * kSortThreads;
+    }
+    const uint32_t n = runs.count;
+    for (uint32_t i = 0; i < n;) {
+        const uint32_t q = __builtin_amdgcn_readfirstlane(runs.run[i]) >> 16;
+        uint64_t w[kSortPer];
+#pragma unroll
+        for (unsigned k = 0; k < kSortPer; ++k)
+            w[k] = from[k] < count ? src[from[k]].w[q] : 0;
+        for (; i < n; ++i) { // the runs within word q
+            const uint32_t e = __builtin_amdgcn_readfirstlane(runs.run[i]);
+            if (e >> 16 != q)
+                break;
+            const uint32_t low = (e >> 8) & 255, bits = e & 255;
+#pragma unroll
+            for (unsigned k = 0; k < kSortPer; ++k)
+                v[k] = v[k] << bits | ((w[k] >> low) & ((1ull << bits) - 1));
+        }
+    }
+#pragma unroll
+    for (unsigned k = 0; k < kSortPer; ++k) {
+        const uint32_t at = threadIdx.x + k * kSortThreads;
+        sh[at] = (from[k] < count ? v[k] : (1ull << kWindow) - 1) << kIndexBits | at;
+    }
+}
+
+// the words by length (8 bits) and the 43 bits below the highest set one
+__device__ __forceinline__ void words_by_length(uint64_t* sh, const Key* __restrict__ src, uint32_t count)
+{
+    for (uint32_t k = threadIdx.x; k < kSortTile; k += kSortThreads) {
+        uint64_t v = (1ull << kWindow) - 1;
+        if (k < count) {
+            const Key x = key_load(src + k);
+            uint64_t top = x.w[0], below = 0, words = 0;
+#pragma unroll
+            for (int q = 1; q < 4; ++q)
+                if (x.w[q]) {
+                    top = x.w[q];
+                    below = x.w[q - 1];
+                    words = q;
+                }
+            const uint32_t zeros = top ? __builtin_clzll(top) : 64;
+            if (zeros < 64 && zeros)
+                top = top << zeros | below >> (64 - zeros);
+            v = (64 * (words + 1) - zeros) << 43 | (top << 1) >> 21;
+        }
+        sh[k] = v << kIndexBits | k;
+    }
+}
+
 __global__ void __launch_bounds__(kSortThreads) tile_sort_kernel(const Key* __restrict__ keys,
     Key* __restrict__ out, uint64_t U, uint64_t stride)
 {
     __shared__ uint64_t sh[kSortTile];
     __shared__ uint16_t perm[kSortTile];
-    __shared__ unsigned long long differ[4];
-    __shared__ uint32_t tie;
+    __shared__ unsigned long long differ[4]; // bits in which the keys differ
+    __shared__ unsigned long long tell[4]; // highest differing bits of neighbours
+    __shared__ uint32_t unsure[4]; // the look at neighbours, then the checks
+    __shared__ BitRuns runs;
     const uint64_t base = (uint64_t)blockIdx.x * kSortTile;
     const Key* src = keys + blockIdx.y * stride + base;
     Key* dst = out + blockIdx.y * stride + base;
     const uint32_t count = U - base < kSortTile ? (uint32_t)(U - base) : kSortTile;
     const uint32_t t = threadIdx.x;
-    if (t < 4)
+    if (t < 4) {
         differ[t] = 0;
-    if (t == 0)
-        tie = 0;
+        tell[t] = 0;
+        unsure[t] = 0;
+    }
     __syncthreads();
+    // into[q] |= x[q] of all threads
+    auto gather = [t](unsigned long long* into, uint64_t (&x)[4]) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            for (int d = 32; d; d >>= 1)
+                x[q] |= __shfl_xor(x[q], d, 64);
+            if ((t & 63) == 0 && x[q])
+                atomicOr(&into[q], (unsigned long long)x[q]);
+        }
+    };
     const Key first = key_load(src);
     uint64_t x[4] = { 0, 0, 0, 0 };
     for (uint32_t k = t; k < count; k += kSortThreads) {
@@ -244,58 +373,166 @@ __global__ void __launch_bounds__(kSortThreads) tile_sort_kernel(const Key* __re
         for (int q = 0; q < 4; ++q)
             x[q] |= v.w[q] ^ first.w[q];
     }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        for (int d = 32; d; d >>= 1)
-            x[q] |= __shfl_xor(x[q], d, 64);
-        if ((t & 63) == 0 && x[q])
-            atomicOr(&differ[q], (unsigned long long)x[q]);
-    }
+    gather(differ, x);
     __syncthreads();
     uint32_t bits = 0; // the keys differ in bits below this one only
     for (int q = 3; q >= 0 && !bits; --q)
         if (differ[q])
             bits = 64 * q + 64 - __builtin_clzll(differ[q]);
     const uint32_t shift = bits > kWindow ? bits - kWindow : 0;
-    // padding sorts last: its words have every window bit set, and its places are past the keys'
-    for (uint32_t k = t; k < kSortTile; k += kSortThreads)
-        sh[k] = ((k < count ? key_window(src + k, shift) : (1ull << kWindow) - 1) << kIndexBits) | k;
-    sort_words(sh);
-    if (shift) {
+    const uint64_t all[4] = { differ[0], differ[1], differ[2], differ[3] };
+    const bool few = bits_set(all) <= kWindow;
+
+    // Chooses the bits that tell keys apart, of the order that sh gives or (sorted false) of the
+    // tile's own; false if they are too many.
+    auto choose = [&](bool sorted) -> bool {
+        uint64_t y[4] = { 0, 0, 0, 0 };
         for (uint32_t k = t; k + 1 < count; k += kSortThreads) {
-            const uint64_t a = sh[k], b = sh[k + 1];
-            if ((a ^ b) >> kIndexBits == 0
-                && !key_eq(key_load(src + (a & kIndexMask)), key_load(src + (b & kIndexMask))))
-                tie = 1;
-        }
-    }
-    __syncthreads();
-    if (tie) { // the same for the whole work-group
-        for (uint32_t k = t; k < kSortTile; k += kSortThreads)
-            perm[k] = (uint16_t)k;
-        for (uint32_t lo = 0; lo < bits; lo += kWindow) {
-            __syncthreads();
-            for (uint32_t k = t; k < kSortTile; k += kSortThreads) {
-                const uint32_t i = perm[k];
-                sh[k] = ((i < count ? key_window(src + i, lo) : (1ull << kWindow) - 1) << kIndexBits) | k;
+            const Key a = key_load(src + (sorted ? sh[k] & kIndexMask : k));
+#pragma unroll
+            for (uint32_t pair = 0; pair < 3; ++pair) { // the next one, the one after it, one near
+                const uint32_t other = pair == 0 ? k + 1 : pair == 1 ? k + 2 : near_to(k, count);
+                if (other >= count || (sorted && pair))
+                    break;
+                const Key b = key_load(src + (sorted ? sh[other] & kIndexMask : other));
+                bool above = false;
+#pragma unroll
+                for (int q = 3; q >= 0; --q) {
+                    const uint64_t e = above ? 0 : a.w[q] ^ b.w[q];
+                    y[q] |= e ? 1ull << (63 - __builtin_clzll(e)) : 0;
+                    above = above || e;
+                }
             }
-            sort_words(sh);
-            uint16_t next[kSortPer];
-#pragma unroll
-            for (unsigned k = 0; k < kSortPer; ++k)
-                next[k] = perm[sh[t + k * kSortThreads] & kIndexMask];
-            __syncthreads();
-#pragma unroll
-            for (unsigned k = 0; k < kSortPer; ++k)
-                perm[t + k * kSortThreads] = next[k];
+        }
+        gather(tell, y);
+        __syncthreads();
+        uint64_t m[4] = { tell[0], tell[1], tell[2], tell[3] };
+        const bool fits = bits_set(m) <= kWindow - 13; // leaves some to the bits below them
+        if (fits && t < 64) { // lane e: the bits and the e below each; the most that fit are taken
+            uint32_t w = 1;
+            for (; 2 * w <= t + 1; w *= 2)
+                or_shifted(m, w);
+            if (w < t + 1)
+                or_shifted(m, t + 1 - w);
+            if (63u - __builtin_clzll(__ballot(bits_set(m) <= kWindow)) == t)
+                set_runs(runs, m);
         }
         __syncthreads();
-        for (uint32_t k = t; k < count; k += kSortThreads)
-            key_store(dst + k, key_load(src + perm[k]));
-        return;
+        return fits;
+    };
+
+    bool window = false, by_length = false;
+    uint32_t tries = 0;
+    // new words: by bits that tell the keys apart, or by length if there are too many
+    auto retry = [&](bool sorted) {
+        window = false;
+        ++tries;
+        by_length = !choose(sorted);
+        if (by_length)
+            words_by_length(sh, src, count);
+        else
+            words_by_runs(sh, src, count, runs);
+    };
+    if (shift && few) {
+        if (t == 0)
+            set_runs(runs, all);
+        __syncthreads();
+        words_by_runs(sh, src, count, runs);
+    } else {
+        // padding sorts last: its words have every window bit set, and its places are past the keys'
+        window = true;
+        for (uint32_t k = t; k < kSortTile; k += kSortThreads) {
+            const uint64_t v = k < count ? key_window(src + k, shift) : (1ull << kWindow) - 1;
+            sh[k] = v << kIndexBits | k;
+        }
+        if (shift) {
+            __syncthreads();
+            for (uint32_t k = t; k + 1 < count; k += kSortThreads) {
+                const uint32_t other = near_to(k, count);
+                if ((sh[k] ^ sh[other]) >> kIndexBits == 0 && !key_eq(key_load(src + k), key_load(src + other)))
+                    unsure[0] = 1;
+            }
+            __syncthreads();
+            if (unsure[0]) // the same for the whole work-group
+                retry(false);
+        }
     }
+    for (int check = 1;; ++check) {
+        sort_words(sh);
+        const bool complete = few || shift == 0;
+        if (window && !complete) {
+            for (uint32_t k = t; k + 1 < count; k += kSortThreads) {
+                const uint64_t a = sh[k], b = sh[k + 1];
+                if ((a ^ b) >> kIndexBits == 0 && key_lt(key_load(src + (b & kIndexMask)), key_load(src + (a & kIndexMask))))
+                    unsure[check] = 1;
+            }
+            __syncthreads();
+        }
+        if (!window || !unsure[check]) { // the output; with chosen bits it is checked as it is written
+            for (uint32_t k = t; k < kSortTile; k += kSortThreads) {
+                Key v {}, before {};
+                if (k < count)
+                    v = key_load(src + (sh[k] & kIndexMask));
+                if (!window && !complete) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        before.w[q] = __shfl_up(v.w[q], 1, 64);
+                    if ((t & 63) == 0 && k && k < count)
+                        before = key_load(src + (sh[k - 1] & kIndexMask));
+                    if (k && k < count && key_lt(v, before))
+                        unsure[check] = 1;
+                }
+                if (k < count)
+                    key_store(dst + k, v);
+            }
+        }
+        if (complete)
+            return;
+        if (!window)
+            __syncthreads();
+        if (!unsure[check])
+            return;
+        if (by_length || tries == 2)
+            break;
+        retry(true);
+    }
+    // by all the bits in which keys differ, 51 at a time
+    __syncthreads();
+    for (uint32_t k = t; k < kSortTile; k += kSortThreads)
+        perm[k] = (uint16_t)k;
+    uint64_t rest[4] = { all[0], all[1], all[2], all[3] };
+    while (bits_set(rest)) {
+        __syncthreads();
+        if (t == 0) {
+            uint64_t m[4] = { 0, 0, 0, 0 };
+            uint32_t n = 0;
+            for (int q = 0; q < 4; ++q)
+                for (; rest[q] && n < kWindow; ++n) {
+                    const uint64_t low = rest[q] & (0 - rest[q]);
+                    m[q] |= low;
+                    rest[q] ^= low;
+                }
+            set_runs(runs, m);
+            for (int q = 0; q < 4; ++q)
+                tell[q] = rest[q];
+        }
+        __syncthreads();
+        for (int q = 0; q < 4; ++q)
+            rest[q] = tell[q];
+        words_by_runs(sh, src, count, runs, perm);
+        sort_words(sh);
+        uint16_t next[kSortPer];
+#pragma unroll
+        for (unsigned k = 0; k < kSortPer; ++k)
+            next[k] = perm[sh[t + k * kSortThreads] & kIndexMask];
+        __syncthreads();
+#pragma unroll
+        for (unsigned k = 0; k < kSortPer; ++k)
+            perm[t + k * kSortThreads] = next[k];
+    }
+    __syncthreads();
     for (uint32_t k = t; k < count; k += kSortThreads)
-        key_store(dst + k, key_load(src + (sh[k] & kIndexMask)));
+        key_store(dst + k, key_load(src + perm[k]));
 }
 
 // Geometry of output tile `tile` in a merge pass over runs of length w: the

@@ -116,3 +116,44 @@ def test_permute_sort_windows(lib, co, U, pattern):
     permute_expression_pair_device(dv.to_device(inp), dv.to_device(table), d_pi, d_pt, U, U)
     assert (dv.to_host(d_pi) == exp_i).all()
     assert (dv.to_host(d_pt) == exp_t).all()
+
+
+@pytest.mark.parametrize("U", [5, 1023, 8191, 8193, 3 * 8192 + 1])
+@pytest.mark.parametrize("pattern", ["signed", "signed_wide", "three_groups", "packed", "powers", "groups_of_many", "late_tie",
+                                     "two_ends"])
+def test_permute_sort_bit_choices(lib, co, U, pattern):
+    """Columns for every way in which a tile finds the bits that order its keys: signed numbers
+    (small and 100 bits), three far groups, packed bytes and two values (few differing bits),
+    powers of two (lengths), many lengths with long rests (all bits in turn), and a tie in the
+    window that no two neighbours of the input show."""
+    from halo2_amd import device as dv
+    from halo2_amd.fields import R_MOD, mont_limbs
+    from halo2_amd.lookup import permute_expression_pair_device
+
+    rng = np.random.default_rng(U)
+
+    def wide(bits):
+        return [int.from_bytes(rng.bytes(32), "little") >> (256 - bits) for _ in range(U)]
+
+    if pattern in ("signed", "signed_wide"):
+        vals = [v if v & 1 else -v for v in wide(12 if pattern == "signed" else 100)]
+    elif pattern == "three_groups":
+        vals = [v + (g % 3) * (R_MOD // 2 - 1500) for v, g in zip(wide(11), wide(8))]
+    elif pattern == "packed":
+        vals = [sum((v >> (8 * j) & 255) << (61 * j) for j in range(4)) for v in wide(32)]
+    elif pattern == "powers":
+        vals = [1 << (v % 254) for v in wide(16)]
+    elif pattern == "groups_of_many":
+        vals = [(1 << (253 - v % 40)) + w for v, w in zip(wide(16), wide(100))]
+    elif pattern == "late_tie":
+        vals = wide(253)
+        vals[0], vals[-1], vals[U // 2] = vals[1] ^ 5, vals[1] ^ 3, vals[1] ^ (1 << 150)
+    else:
+        vals = [0 if v & 1 else R_MOD - 1 for v in wide(8)]
+    table = np.stack([mont_limbs(v % R_MOD) for v in vals])
+    inp = table[rng.integers(0, U, U)]
+    exp_i, exp_t = co.permute_expression_pair(inp, table, U, U)
+    d_pi, d_pt = dv.empty_u64(4 * U), dv.empty_u64(4 * U)
+    permute_expression_pair_device(dv.to_device(inp), dv.to_device(table), d_pi, d_pt, U, U)
+    assert (dv.to_host(d_pi) == exp_i).all()
+    assert (dv.to_host(d_pt) == exp_t).all()
