@@ -54,7 +54,10 @@ constexpr uint32_t R1_TILE = R1_THREADS * R1_PER; // points per round-1 tile
 constexpr uint32_t R2_THREADS = 1024;
 constexpr uint32_t R2_CHUNK = 16384; // entries per round-2 chunk (staged in LDS)
 constexpr uint32_t LIGHT = 8; // pieces of a split bucket that one quad sums, more than twice the average bucket's
-constexpr uint32_t HEAVY_THREADS = 256;
+// A work-group per dense bucket: with 64 quads the 65 536 pieces of a bucket that holds every digit of
+// a window (2^20 equal scalars) were 1024 additions deep, and a table MSM of them took 3.75 ms, with
+// 128 3.22; half as many work-groups cost 131 072 points 26 us.
+constexpr uint32_t HEAVY_THREADS = 512;
 constexpr uint32_t HEAVY_BLOCKS = 512;
 constexpr uint32_t RED_L1 = 16; // at most this many buckets per first-level reduction segment
 constexpr uint64_t RED_THREADS = 1ull << 17; // first-level segments wanted: 2 waves per SIMD
