@@ -413,9 +413,11 @@ struct F29 {
 
     // The same value as pow_m_minus_2 (u^-1 * 2^261 for a = u * 2^261, i.e.
     // 2^522 / A for the integer A = a mod m; zero maps to zero) by
-    // division steps (inv_mod_plain) and one product with 2^783, called by one lane of a
-    // wave only. Input normalised, < 2m; output a normalised representative < 1.01m.
-    __device__ static F29 inverse_vt(const F29 a)
+    // division steps (inv_mod_plain) and one product with 2^783. For one active lane of the wave:
+    // the steps are in scalar registers, so other lanes would get the first one's inverse
+    // (Fp256::inverse_vt is the form for any lanes). Input normalised, < 2m; output a
+    // normalised representative < 1.01m.
+    __device__ static F29 inverse_one_lane(const F29 a)
     {
         const F29 c = reduce_full(a);
         if (c.is_zero())

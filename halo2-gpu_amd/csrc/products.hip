@@ -100,7 +100,7 @@ __global__ void __launch_bounds__(T) batch_invert_kernel(uint8_t* __restrict__ d
     if (tid == 0) {
         F k251 = F::zero();
         k251.l[8] = 1u << 19; // 2^251 = 2^(232 + 19)
-        node[1] = F::mul(F::inverse_vt(node[1]), k251);
+        node[1] = F::mul(F::inverse_one_lane(node[1]), k251);
     }
     __syncthreads();
     // inverse of this thread's product
@@ -364,7 +364,7 @@ __global__ void __launch_bounds__(kMidThreads) totals_inverse_kernel(A acc_total
     if (tid == 0) {
         F k251 = F::zero();
         k251.l[8] = 1u << 19; // 2^251 = 2^(232 + 19)
-        inv_all = F::mul(F::inverse_vt(pre[kMidThreads - 1]), k251);
+        inv_all = F::mul(F::inverse_one_lane(pre[kMidThreads - 1]), k251);
     }
     __syncthreads();
     F inv = inv_all;
