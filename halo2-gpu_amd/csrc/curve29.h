@@ -190,18 +190,6 @@ struct G1X29 {
         const Fq29 zz = Fq29::sqr(jz);
         return G1X29 { jx, jy, zz, Fq29::mul(zz, jz) };
     }
-
-    // back to the 2^256 scale (canonical) for the final affine conversion
-    __device__ G1Xyzz to_xyzz256() const
-    {
-        const Fq29 f = Fq29::from_limbs(Fq29P::FROM261);
-        G1Xyzz r;
-        Fq29::reduce_full(Fq29::mul(X, f)).to32(r.X.v);
-        Fq29::reduce_full(Fq29::mul(Y, f)).to32(r.Y.v);
-        Fq29::reduce_full(Fq29::mul(ZZ, f)).to32(r.ZZ.v);
-        Fq29::reduce_full(Fq29::mul(ZZZ, f)).to32(r.ZZZ.v);
-        return r;
-    }
 };
 
 } // namespace h2

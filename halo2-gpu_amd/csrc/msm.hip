@@ -1651,7 +1651,6 @@ __global__ void ec_affine_kernel(const PointSlot* __restrict__ P, const uint32_t
 
 unsigned blocks_for(uint64_t n, unsigned t) { return (unsigned)((n + t - 1) / t); }
 
-uint32_t ilog2(uint32_t x) { return 31 - __builtin_clz(x); }
 
 // Full device pipeline; the window sums land in b.out (device, for finish_on_host). A batch
 // (p.batch) has its canonical scalars and job tables in place already and

@@ -91,17 +91,22 @@ static void host_limbs(const uint32_t (&w)[8], uint32_t (&l)[9])
     l[8] = w[7] >> 8;
 }
 
-// Output scale s (one for POST_NONE): s 2^290 mod r, and 2^29 s 8 K mod r, K = sum_b 128 2^(8b),
-// the part of a radix-8 last step's y_0 that the shift of the data bytes takes away
-// (ntt_mfma.h; a radix-16 step's is twice that)
-static void host_scale290(NttPost post, const Fr& scale, uint32_t (&limbs)[9], uint32_t (&bias8)[9])
+// Output scale s (one for POST_NONE): s 2^290 mod r
+static void host_scale290(NttPost post, const Fr& scale, uint32_t (&s)[8])
 {
-    static constexpr uint32_t k8k[8] = { 0x20202020u, 0x20202020u, 0x20202020u, 0x20202020u, 0x20202020u, 0x20202020u, 0x20202020u, 0x20202020u }; // 8 K / 2^5
-    uint32_t s[8], b[8];
     host_mont_mul(post == POST_NONE ? FrParams::ONE : scale.v, kTo290, s);
+}
+
+// 2^29 s 8 K mod r, K = sum_b 128 2^(8b): the part of a radix-8 last step's y_0 that the shift of
+// the data bytes takes away (ntt_mfma.h; a radix-16 step's is twice that)
+static void host_bias8(NttPost post, const Fr& scale, uint32_t (&limbs)[9])
+{
+    static constexpr uint32_t k8k[8] = { 0x20202020u, 0x20202020u, 0x20202020u, 0x20202020u, 0x20202020u, 0x20202020u,
+        0x20202020u, 0x20202020u }; // 8 K / 2^5
+    uint32_t s[8], b[8];
+    host_scale290(post, scale, s);
     host_mont_mul(s, k8k, b);
-    host_limbs(s, limbs);
-    host_limbs(b, bias8);
+    host_limbs(b, limbs);
 }
 
 // The direct DFT's last factors for output index i mod 3: s zeta^-(i mod 3)
@@ -284,12 +289,7 @@ __global__ void __launch_bounds__(64) ntt_tables_kernel(TableSets sets)
             r.l[k] = (x >> s) & 1 ? m.l[k] : r.l[k];
     }
     if (job.kind == TABLE_UNIT) {
-        Fr29 one256;
-#pragma unroll
-        for (int k = 0; k < 9; ++k)
-            one256.l[k] = 0;
-        Fr one = Fr::one(); // 2^256 mod m: back from the 2^261 scale
-        one256 = Fr29::from_fp(one);
+        const Fr29 one256 = Fr29::from_fp(Fr::one()); // 2^256 mod m: back from the 2^261 scale
         uint32_t w[8];
         Fr29::reduce_full(Fr29::mul(r, one256)).to32(w);
         bool same = true;
@@ -336,8 +336,9 @@ RustError ntt_tables_plan(Workspace& ws, NttTables& t, uint32_t log_n, const Fr*
     ts.log_n = log_n;
     ts.omega = d_omega;
     ts.c = c;
-    uint32_t bias8[9];
-    host_scale290(post, scale, ts.scale290, bias8);
+    uint32_t scale290[8];
+    host_scale290(post, scale, scale290);
+    host_limbs(scale290, ts.scale290);
     auto job = [&](void* out, uint32_t count, uint32_t shift, bool use_c, TableKind kind, uint32_t row) {
         ts.j[ts.nj++] = TableJob { (Fr*)out, shift, count, kind, use_c, (uint8_t)row };
     };
@@ -436,7 +437,7 @@ struct PassParams {
     int post;
     int last;
     uint32_t xcd_remap;
-    uint32_t bias8[9]; // of the last step's y_0 (host_scale290)
+    uint32_t bias8[9]; // of the last step's y_0 (host_bias8)
     uint32_t pc[3][9]; // constants of the direct DFT's last product (host_post)
 };
 
@@ -864,9 +865,9 @@ RustError ntt_run(const NttTables& t, uint32_t log_n, const NttJob* jobs, int co
     int max_batch = NTT_MAX_BATCH;
     if (need_scratch && scratch_slots < (uint64_t)max_batch)
         max_batch = (int)scratch_slots;
-    uint32_t pc[3][9], scale290[9], bias8[9];
+    uint32_t pc[3][9], bias8[9];
     host_post(post, scale, pc);
-    host_scale290(post, scale, scale290, bias8);
+    host_bias8(post, scale, bias8);
 
     for (int base = 0; base < count; base += max_batch) {
         const int nb = count - base < max_batch ? count - base : max_batch;
@@ -955,9 +956,9 @@ RustError ntt_run_batch(const NttBatchJob* jobs, int count, NttTwist twist, NttP
         H2_CHECK_ARG(p.P < 3 || jb.scratch, "NTT batch: 2^%u needs a scratch buffer", jb.log_n);
         H2_CHECK_ARG(p.P != 2 || (const void*)jb.in != (const void*)jb.out, "NTT batch: in-place 2^%u transform",
             jb.log_n);
-        uint32_t pc[3][9], scale290[9], bias8[9];
+        uint32_t pc[3][9], bias8[9];
         host_post(post, jb.scale, pc);
-        host_scale290(post, jb.scale, scale290, bias8);
+        host_bias8(post, jb.scale, bias8);
         for (int pass = 0; pass < p.P; ++pass) {
             BatchPass bp {};
             if (p.P == 1) {
