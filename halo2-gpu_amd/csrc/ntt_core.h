@@ -60,7 +60,9 @@ struct NttTables {
 // Workspace bytes for the tables of one transform size (+ optional c tables).
 void ntt_tables_size(WorkspaceSizer& ws, uint32_t log_n, bool powers_twist);
 
-// What one transform's tables are made from: `d_omega` is a device pointer to omega, `c` the
+// What one transform's tables are made from: `d_omega` is a device pointer to omega, a primitive
+// 2^log_n-th root of unity (the steps use omega^(N / 2) = -1 and take their matrices by the 16th root
+// that omega^(N / 16) is; another omega gives no defined result from 2^NTT_MATRIX_LOG points on), `c` the
 // CosetFFT_Part factor (used only with powers_twist), `scale` the output's factor (POST_SCALE*).
 struct NttTableSpec {
     uint32_t log_n;

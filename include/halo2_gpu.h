@@ -92,6 +92,10 @@ RustError h2amd_multiexp_device_scalars_device_bases_noalloc(const void* d_scala
 
 /* ================================================================ NTT */
 
+/* In every transform omega is a primitive root of unity of the transform's size (2^log_n, or
+ * 2^extend_log_n where the output is extended): sums over halves use omega^(size / 2) = -1. With
+ * another omega the output is not defined (below 2^6 points it is the sum by definition). */
+
 /* culib.rs:492 ; cuda/src/ntt.cu:383-393 */
 uint64_t _halo2_fft_normal_workspace_size(uint32_t ntt_type, uint32_t log_n, uint32_t extend_log_n);
 /* culib.rs:494-504 ; ntt.cu:395-474 — host input/output/omega/divisor; FFT, iFFT, cosetFFT,
