@@ -430,16 +430,15 @@ uint64_t plan_bytes(const MsmPlan& p)
 
 // Scratch for n points. Without a table the width follows n, and fewer points at a narrower
 // width can take more (more windows), so it is the most that n points or the last length below
-// each power of two up to 2^18 take. (From 2^19 points on a scratch serves the length it was
-// sized for only.)
+// n's power of two take, up to 2^19 points. (Above, a scratch serves the length it was sized for.)
 uint64_t msm_workspace_bytes(uint64_t n, uint64_t table_n = 0)
 {
-    uint64_t most = plan_bytes(make_plan(n, table_n));
-    for (uint32_t k = 1; !table_n && k <= 18 && (1ull << k) <= n; ++k) {
-        const uint64_t bytes = plan_bytes(make_plan((1ull << k) - 1));
-        most = bytes > most ? bytes : most;
-    }
-    return most;
+    const uint64_t bytes = plan_bytes(make_plan(n, table_n));
+    const uint32_t k = log2_floor(n);
+    if (table_n || k == 0 || k > 18)
+        return bytes;
+    const uint64_t below = plan_bytes(make_plan((1ull << k) - 1));
+    return below > bytes ? below : bytes;
 }
 
 // ------------------------------------------------------------- kernels
@@ -1966,13 +1965,13 @@ uint64_t h2amd_multiexp_batch_workspace_size(const uint64_t* lengths, uint32_t c
         return 0;
     // as msm_workspace_bytes: the width follows the mean length
     const MsmPlan p = make_batch_plan(lengths, count);
-    uint64_t most = plan_bytes(p);
-    for (uint32_t k = 1; k <= 20 && ((uint64_t)count << k) <= p.n; ++k) {
-        const uint64_t nv = (((uint64_t)count << k) - 1) / R1_TILE * R1_TILE;
-        const uint64_t bytes = plan_bytes(batch_plan(nv, p.nbase, count, 0));
-        most = bytes > most ? bytes : most;
-    }
-    return most;
+    const uint64_t bytes = plan_bytes(p);
+    const uint32_t k = log2_floor(p.n / count);
+    if (k == 0 || k > 20)
+        return bytes;
+    const uint64_t nv = (((uint64_t)count << k) - 1) / R1_TILE * R1_TILE;
+    const uint64_t below = plan_bytes(batch_plan(nv, p.nbase, count, 0));
+    return below > bytes ? below : bytes;
 }
 
 // J MSMs in one pipeline over shared bases (table_n = 0) or one precomputed table
