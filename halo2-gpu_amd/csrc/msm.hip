@@ -135,12 +135,12 @@ uint32_t default_width(uint64_t n, bool shared, uint32_t bits)
     int c = (int)log2_floor(n < 1 ? 1 : n) - (shared ? 0 : 4);
     if (c < 4)
         c = 4;
-    if (c > 20) // shared buckets too: measured 2^22 tables 7.6 ms at 20 bits vs 8.3 at 22, 2^24 equal
+    if (c > 20) // shared buckets too: 2^22 tables 5.39 ms at 20 bits, 5.70 at 22
         c = 20;
-    if (!shared && c > 19) // plain 2^24: 26.4 ms at 19 bits (14 windows) vs 27.2 at 20 (13 windows)
+    if (!shared && c > 19) // plain 2^24: 22.6 ms at 19 bits (14 windows), 23.0 at 20 (13 windows)
         c = 19;
     if (shared && c == 20 && n < (1ull << 21)) // 2^20 tables: 15 rows of 17 bits, an eighth of the
-        c = 17; // buckets to reduce: 2.21 vs 2.28 ms per MSM, a k = 20 proof 42.0 vs 43.7 ms
+        c = 17; // buckets to reduce: 1.58 ms per MSM, 1.68 at 20 bits
     // same window count, narrowest width: the top window is as full as the others
     const uint32_t w0 = (bits + (uint32_t)c - 1) / (uint32_t)c;
     return (bits + w0 - 1) / w0;
@@ -172,12 +172,12 @@ uint32_t plain_msm_width(uint64_t npoints)
         return tuned;
     if (!use_glv(npoints))
         return default_width(npoints, false, 255);
-    // GLV from 2^19 points: one bit narrower than the rule (the tuner measured 2^20 at
-    // c = 16: 3.82 ms against 4.23 ms at c = 17; 2^16..2^18 are within noise of the rule)
+    // GLV from 2^19 points: 2^20 takes 1.97 ms at c = 16, 2.08 at the rule's 17 (2^19 has the
+    // rule's 15 here: 1.23 ms, 1.15 at 16; 2^15..2^17 are within 4% of the best at the rule's)
     if (npoints >= (1ull << 19))
         return log2_floor(2 * npoints) - 5;
-    // 2^18 points: 1.30 ms at c = 16 against 1.54 at the rule's 15 (9 windows either way,
-    // but half as many entries per bucket to merge)
+    // 2^18 points: 0.75 ms at c = 16, 0.79 at the rule's 15 (9 windows either way, but half as
+    // many entries per bucket to merge)
     if (npoints >= (1ull << 18))
         return 16;
     return default_width(2 * npoints, false, GLV_BITS);
