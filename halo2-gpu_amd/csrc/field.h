@@ -76,7 +76,8 @@ __host__ __device__ constexpr int32_t modulus30(int i)
 // x^-1 = +-d. 590 steps (20 rounds) reach it for inputs below 2^256; the loop's own limit of 25 is
 // what bounds it. |d|, |e| grow by at most m / 2 a round.
 //
-// Within a round several steps are taken at once: with theta = delta - 1/2, the trailing zeros
+// Within a round several steps are taken at once, in the way that P. Wuille's note "The safegcd
+// implementation in libsecp256k1 explained" (2021) describes for public data: with theta = delta - 1/2, the trailing zeros
 // of g are that many steps at once, and as long as theta < 0 the steps only add f to g, so
 // w = -g / f mod 2^k clears k <= -theta bits by one multiple of f. When theta >= 0 and g is
 // odd, f and g are exchanged (g' = -f, theta' = -theta - 1), and the step is one of adding.

@@ -1,7 +1,7 @@
 """The scalar modular inversion (field.h inv_mod_plain, batched division steps),
 built for the host from the same source and checked against Python's pow(x, -1, m) for
-both BN254 moduli: edge values (1, 2, m - 1, powers of two around the 64-bit
-approximation's boundaries, values just below m) and random ones of every length."""
+both BN254 moduli: edge values (1, 2, m - 1, powers of two around word
+boundaries, values just below m) and random ones of every length."""
 import pathlib
 import random
 import shutil

@@ -53,6 +53,17 @@ def test_column_sums_of_scaled_matrices(seed):
                 assert int(sums.max()) * 257 < 1 << 31
 
 
+@pytest.mark.parametrize("k", range(0, 29))
+def test_column_sums_of_inverse_transforms(k):
+    """The scales that the transforms themselves use, 1 and every 2^-k: the sums fit for certain."""
+    s = pow(2, -k, M)
+    cols = [[pow(G16, e, M) * s * pow(2, 29, M) * pow(256, b, M) % M for b in range(32)] for e in range(16)]
+    digits = np.abs(np.array([[_digits(v if 2 * v <= M else v - M) for v in row] for row in cols]))
+    for r in (16, 8):
+        for j in range(r):
+            assert int(digits[[a * j * (16 // r) % 16 for a in range(r)]].sum(axis=(0, 1)).max()) * 128 * 257 < 1 << 31
+
+
 def test_dft_by_digits(matrices):
     """The steps' arithmetic in Python integers: shifted bytes through the matrices, the shift
     given back to y_0 only, against the DFT itself."""
