@@ -139,24 +139,24 @@ __device__ __forceinline__ void merge_run(const Key* A, uint32_t na, const Key* 
 // place in the tile, four times less to move through LDS and registers; the keys themselves
 // are read where they lie and written once, in order. Which 51 bits:
 //  - the tile's keys differ in 51 bits at most: those, and the order is complete;
-//  - otherwise the window below the highest bit in which they differ. It is checked: the keys of
-//    neighbours that agree in it are compared. For uniform keys it holds but for 2^-26 a tile;
-//  - if it does not hold, which a look at neighbouring keys mostly shows before the sort (signed
-//    small numbers: m - x and x share all the window), the bits that tell keys apart. The highest
-//    bit in which two keys differ, for every two neighbours of a sorted order, is enough to
-//    compare any two keys; neighbours of an unsorted order give most of these bits, and the ones
-//    right below them, as far as 51 reach, the rest. All neighbours' keys are then compared;
+//  - otherwise the window below the highest bit in which they differ. Neighbours that agree in it
+//    are then compared; for uniform keys they are equal but for 2^-26 a tile;
+//  - if a look at neighbouring keys before the sort shows a window that ties (signed small numbers:
+//    m - x and x share all of it), the bits that tell keys apart. The highest bit in which two
+//    keys differ, for every two neighbours of a sorted order, is enough to compare any two keys;
+//    neighbours of an unsorted order give most of these bits, and the ones right below them, as
+//    far as 51 reach, the rest. The order is checked as the keys are written;
 //  - if there are too many such bits, the keys' lengths vary (powers of two, say): the length and
-//    the 43 bits below the highest one, checked in the same way;
-//  - after that, or two rounds of chosen bits, the tile is sorted by all the bits in which its keys
-//    differ, 51 a round and the lowest first (the place in the current order keeps each round stable).
+//    the 43 bits below the highest one.
+// Keys that a window or a length leaves tied go through further rounds of their rank so far and 38
+// of the bits in which tied keys differ.
 // Words are sorted 8 per thread in registers, then in ten merge rounds.
-// 2^20 rows of two columns: 213 us with keys as the words and 2048 a tile, now 85, and two
+// 2^20 rows of two columns: 213 us with keys as the words and 2048 a tile, now 88, and two
 // merge passes of 38 us less. The whole call for signed numbers, 2^10, 2^16 and 2^20 rows: 92,
-// 188, 713 us with keys as the words, now 75, 158, 603 (263, 360, 754 if a tile that ties in its
-// window goes through all of them); for powers of two 91, 183, 683 and now 74, 156, 510. Keys that
-// need all the bits (40 lengths with more than 43 bits below) take longer: 88, 175, 671 and 239,
-// 362, 772.
+// 188, 713 us with keys as the words, now 75, 158, 639 (263, 360, 754 if a tile that ties in its
+// window goes through all of them); for powers of two 91, 183, 678 and now 73, 164, 528. Keys that
+// need a second round (40 lengths with more than 43 bits below) take longer on few rows: 88, 175,
+// 669 and now 120, 218, 595.
 constexpr unsigned kSortThreads = 1024;
 constexpr unsigned kSortPer = kSortTile / kSortThreads;
 constexpr unsigned kIndexBits = 13;
@@ -276,24 +276,23 @@ __device__ __forceinline__ uint32_t near_to(uint32_t k, uint32_t count)
     return other < count ? other : count - 1;
 }
 
-// the words of the tile's keys (in the order `perm`, if any) by a choice of bits
+// the words of the tile's keys by a choice of bits, below their ranks (if any)
 __device__ __forceinline__ void words_by_runs(uint64_t* sh, const Key* __restrict__ src, uint32_t count,
-    const BitRuns& runs, const uint16_t* perm = nullptr)
+    const BitRuns& runs, const uint16_t* rank = nullptr)
 {
     uint64_t v[kSortPer];
-    uint32_t from[kSortPer];
 #pragma unroll
-    for (unsigned k = 0; k < kSortPer; ++k) {
-        v[k] = 0;
-        from[k] = perm ? perm[threadIdx.x + k * kSortThreads] : threadIdx.x + k * kSortThreads;
-    }
+    for (unsigned k = 0; k < kSortPer; ++k)
+        v[k] = rank ? rank[threadIdx.x + k * kSortThreads] : 0;
     const uint32_t n = runs.count;
     for (uint32_t i = 0; i < n;) {
         const uint32_t q = __builtin_amdgcn_readfirstlane(runs.run[i]) >> 16;
         uint64_t w[kSortPer];
 #pragma unroll
-        for (unsigned k = 0; k < kSortPer; ++k)
-            w[k] = from[k] < count ? src[from[k]].w[q] : 0;
+        for (unsigned k = 0; k < kSortPer; ++k) {
+            const uint32_t at = threadIdx.x + k * kSortThreads;
+            w[k] = at < count ? src[at].w[q] : 0;
+        }
         for (; i < n; ++i) { // the runs within word q
             const uint32_t e = __builtin_amdgcn_readfirstlane(runs.run[i]);
             if (e >> 16 != q)
@@ -307,8 +306,15 @@ __device__ __forceinline__ void words_by_runs(uint64_t* sh, const Key* __restric
 #pragma unroll
     for (unsigned k = 0; k < kSortPer; ++k) {
         const uint32_t at = threadIdx.x + k * kSortThreads;
-        sh[at] = (from[k] < count ? v[k] : (1ull << kWindow) - 1) << kIndexBits | at;
+        sh[at] = (at < count ? v[k] : (1ull << kWindow) - 1) << kIndexBits | at;
     }
+}
+
+// the words by the window from bit `shift` up
+__device__ __forceinline__ void words_by_window(uint64_t* sh, const Key* __restrict__ src, uint32_t count, uint32_t shift)
+{
+    for (uint32_t k = threadIdx.x; k < kSortTile; k += kSortThreads)
+        sh[k] = (k < count ? key_window(src + k, shift) : (1ull << kWindow) - 1) << kIndexBits | k;
 }
 
 // the words by length (8 bits) and the 43 bits below the highest set one
@@ -339,29 +345,31 @@ __global__ void __launch_bounds__(kSortThreads) tile_sort_kernel(const Key* __re
     Key* __restrict__ out, uint64_t U, uint64_t stride)
 {
     __shared__ uint64_t sh[kSortTile];
-    __shared__ uint16_t perm[kSortTile];
+    __shared__ uint16_t rank[kSortTile];
     __shared__ unsigned long long differ[4]; // bits in which the keys differ
-    __shared__ unsigned long long tell[4]; // highest differing bits of neighbours
-    __shared__ uint32_t unsure[4]; // the look at neighbours, then the checks
+    __shared__ unsigned long long tell[4]; // highest differing bits of neighbours; bits in which tied keys differ
+    __shared__ uint32_t last_head[kSortThreads / 64];
+    __shared__ uint32_t ties, misplaced;
     __shared__ BitRuns runs;
     const uint64_t base = (uint64_t)blockIdx.x * kSortTile;
     const Key* src = keys + blockIdx.y * stride + base;
     Key* dst = out + blockIdx.y * stride + base;
     const uint32_t count = U - base < kSortTile ? (uint32_t)(U - base) : kSortTile;
-    const uint32_t t = threadIdx.x;
+    const uint32_t t = threadIdx.x, lane = t & 63;
     if (t < 4) {
         differ[t] = 0;
         tell[t] = 0;
-        unsure[t] = 0;
     }
+    if (t == 0)
+        ties = misplaced = 0;
     __syncthreads();
     // into[q] |= x[q] of all threads
-    auto gather = [t](unsigned long long* into, uint64_t (&x)[4]) {
+    auto gather = [lane](unsigned long long* into, uint64_t (&x)[4]) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             for (int d = 32; d; d >>= 1)
                 x[q] |= __shfl_xor(x[q], d, 64);
-            if ((t & 63) == 0 && x[q])
+            if (lane == 0 && x[q])
                 atomicOr(&into[q], (unsigned long long)x[q]);
         }
     };
@@ -383,18 +391,18 @@ __global__ void __launch_bounds__(kSortThreads) tile_sort_kernel(const Key* __re
     const uint64_t all[4] = { differ[0], differ[1], differ[2], differ[3] };
     const bool few = bits_set(all) <= kWindow;
 
-    // Chooses the bits that tell keys apart, of the order that sh gives or (sorted false) of the
-    // tile's own; false if they are too many.
-    auto choose = [&](bool sorted) -> bool {
+    // Chooses the bits that tell neighbouring keys apart and the ones below them; false if they
+    // are too many.
+    auto choose = [&]() -> bool {
         uint64_t y[4] = { 0, 0, 0, 0 };
         for (uint32_t k = t; k + 1 < count; k += kSortThreads) {
-            const Key a = key_load(src + (sorted ? sh[k] & kIndexMask : k));
+            const Key a = key_load(src + k);
 #pragma unroll
             for (uint32_t pair = 0; pair < 3; ++pair) { // the next one, the one after it, one near
                 const uint32_t other = pair == 0 ? k + 1 : pair == 1 ? k + 2 : near_to(k, count);
-                if (other >= count || (sorted && pair))
+                if (other >= count)
                     break;
-                const Key b = key_load(src + (sorted ? sh[other] & kIndexMask : other));
+                const Key b = key_load(src + other);
                 bool above = false;
 #pragma unroll
                 for (int q = 3; q >= 0; --q) {
@@ -418,121 +426,123 @@ __global__ void __launch_bounds__(kSortThreads) tile_sort_kernel(const Key* __re
                 set_runs(runs, m);
         }
         __syncthreads();
+        if (t < 4)
+            tell[t] = 0;
         return fits;
     };
 
-    bool window = false, by_length = false;
-    uint32_t tries = 0;
-    // new words: by bits that tell the keys apart, or by length if there are too many
-    auto retry = [&](bool sorted) {
-        window = false;
-        ++tries;
-        by_length = !choose(sorted);
-        if (by_length)
-            words_by_length(sh, src, count);
-        else
-            words_by_runs(sh, src, count, runs);
+    // The tile's keys in the words' order; with `check` a key below the one before it sets `misplaced`.
+    auto write = [&](bool check) {
+        for (uint32_t k = t; k < kSortTile; k += kSortThreads) {
+            Key v {}, before {};
+            if (k < count)
+                v = key_load(src + (sh[k] & kIndexMask));
+            if (check) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    before.w[q] = __shfl_up(v.w[q], 1, 64);
+                if (lane == 0 && k && k < count)
+                    before = key_load(src + (sh[k - 1] & kIndexMask));
+                if (k && k < count && key_lt(v, before))
+                    misplaced = 1;
+            }
+            if (k < count)
+                key_store(dst + k, v);
+        }
     };
+
+    // padding sorts last: its words have every window bit set, and its places are past the keys'
     if (shift && few) {
         if (t == 0)
             set_runs(runs, all);
         __syncthreads();
         words_by_runs(sh, src, count, runs);
     } else {
-        // padding sorts last: its words have every window bit set, and its places are past the keys'
-        window = true;
-        for (uint32_t k = t; k < kSortTile; k += kSortThreads) {
-            const uint64_t v = k < count ? key_window(src + k, shift) : (1ull << kWindow) - 1;
-            sh[k] = v << kIndexBits | k;
+        words_by_window(sh, src, count, shift);
+    }
+    if (shift && !few) {
+        __syncthreads();
+        for (uint32_t k = t; k + 1 < count; k += kSortThreads) {
+            const uint32_t other = near_to(k, count);
+            if ((sh[k] ^ sh[other]) >> kIndexBits == 0 && !key_eq(key_load(src + k), key_load(src + other)))
+                ties = 1;
         }
-        if (shift) {
-            __syncthreads();
-            for (uint32_t k = t; k + 1 < count; k += kSortThreads) {
-                const uint32_t other = near_to(k, count);
-                if ((sh[k] ^ sh[other]) >> kIndexBits == 0 && !key_eq(key_load(src + k), key_load(src + other)))
-                    unsure[0] = 1;
+        __syncthreads();
+        if (ties) { // the same for the whole work-group
+            if (choose()) {
+                words_by_runs(sh, src, count, runs);
+                sort_words(sh);
+                write(true);
+                __syncthreads();
+                if (!misplaced)
+                    return;
+                words_by_window(sh, src, count, shift);
+            } else {
+                words_by_length(sh, src, count);
             }
-            __syncthreads();
-            if (unsure[0]) // the same for the whole work-group
-                retry(false);
         }
     }
-    for (int check = 1;; ++check) {
-        sort_words(sh);
-        const bool complete = few || shift == 0;
-        if (window && !complete) {
-            for (uint32_t k = t; k + 1 < count; k += kSortThreads) {
-                const uint64_t a = sh[k], b = sh[k + 1];
-                if ((a ^ b) >> kIndexBits == 0 && key_lt(key_load(src + (b & kIndexMask)), key_load(src + (a & kIndexMask))))
-                    unsure[check] = 1;
-            }
-            __syncthreads();
-        }
-        if (!window || !unsure[check]) { // the output; with chosen bits it is checked as it is written
-            for (uint32_t k = t; k < kSortTile; k += kSortThreads) {
-                Key v {}, before {};
-                if (k < count)
-                    v = key_load(src + (sh[k] & kIndexMask));
-                if (!window && !complete) {
+    sort_words(sh);
+    // The words' bits are in the keys' order now, but keys may share them: the words of the next round
+    // are the place of the first key of each such group and the highest 38 bits in which keys of
+    // a group differ.
+    for (bool exact = few || shift == 0; !exact;) {
+        uint64_t y[4] = { 0, 0, 0, 0 };
+        for (uint32_t k = t; k + 1 < count; k += kSortThreads) {
+            const uint64_t a = sh[k], b = sh[k + 1];
+            if ((a ^ b) >> kIndexBits)
+                continue;
+            const Key ka = key_load(src + (a & kIndexMask)), kb = key_load(src + (b & kIndexMask));
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        before.w[q] = __shfl_up(v.w[q], 1, 64);
-                    if ((t & 63) == 0 && k && k < count)
-                        before = key_load(src + (sh[k - 1] & kIndexMask));
-                    if (k && k < count && key_lt(v, before))
-                        unsure[check] = 1;
-                }
-                if (k < count)
-                    key_store(dst + k, v);
-            }
+            for (int q = 0; q < 4; ++q)
+                y[q] |= ka.w[q] ^ kb.w[q];
         }
-        if (complete)
-            return;
-        if (!window)
-            __syncthreads();
-        if (!unsure[check])
-            return;
-        if (by_length || tries == 2)
+        if (__any((y[0] | y[1] | y[2] | y[3]) != 0))
+            gather(tell, y);
+        __syncthreads();
+        uint64_t m[4] = { tell[0], tell[1], tell[2], tell[3] };
+        if (bits_set(m) == 0)
             break;
-        retry(true);
-    }
-    // by all the bits in which keys differ, 51 at a time
-    __syncthreads();
-    for (uint32_t k = t; k < kSortTile; k += kSortThreads)
-        perm[k] = (uint16_t)k;
-    uint64_t rest[4] = { all[0], all[1], all[2], all[3] };
-    while (bits_set(rest)) {
+        exact = bits_set(m) <= kWindow - kIndexBits;
+        uint32_t head = 0; // of the group that the thread's 8 words end in, then of all before them
+#pragma unroll
+        for (unsigned k = 0; k < kSortPer; ++k) {
+            const uint32_t at = t * kSortPer + k;
+            if (at && (sh[at] ^ sh[at - 1]) >> kIndexBits)
+                head = at;
+        }
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t h = __shfl_up(head, d, 64);
+            head = lane >= (uint32_t)d && h > head ? h : head;
+        }
+        if (lane == 63)
+            last_head[t >> 6] = head;
+        head = __shfl_up(head, 1, 64);
+        if (lane == 0)
+            head = 0;
         __syncthreads();
+        for (uint32_t w = 0; w < t >> 6; ++w)
+            head = last_head[w] > head ? last_head[w] : head;
+#pragma unroll
+        for (unsigned k = 0; k < kSortPer; ++k) {
+            const uint32_t at = t * kSortPer + k;
+            if (at && (sh[at] ^ sh[at - 1]) >> kIndexBits)
+                head = at;
+            rank[sh[at] & kIndexMask] = (uint16_t)head;
+        }
         if (t == 0) {
-            uint64_t m[4] = { 0, 0, 0, 0 };
-            uint32_t n = 0;
-            for (int q = 0; q < 4; ++q)
-                for (; rest[q] && n < kWindow; ++n) {
-                    const uint64_t low = rest[q] & (0 - rest[q]);
-                    m[q] |= low;
-                    rest[q] ^= low;
-                }
+            for (int q = 0; q < 4; ++q) // the lowest bits go
+                while (m[q] && bits_set(m) > kWindow - kIndexBits)
+                    m[q] &= m[q] - 1;
             set_runs(runs, m);
-            for (int q = 0; q < 4; ++q)
-                tell[q] = rest[q];
         }
         __syncthreads();
-        for (int q = 0; q < 4; ++q)
-            rest[q] = tell[q];
-        words_by_runs(sh, src, count, runs, perm);
+        if (t < 4)
+            tell[t] = 0;
+        words_by_runs(sh, src, count, runs, rank);
         sort_words(sh);
-        uint16_t next[kSortPer];
-#pragma unroll
-        for (unsigned k = 0; k < kSortPer; ++k)
-            next[k] = perm[sh[t + k * kSortThreads] & kIndexMask];
-        __syncthreads();
-#pragma unroll
-        for (unsigned k = 0; k < kSortPer; ++k)
-            perm[t + k * kSortThreads] = next[k];
     }
-    __syncthreads();
-    for (uint32_t k = t; k < count; k += kSortThreads)
-        key_store(dst + k, key_load(src + perm[k]));
+    write(false);
 }
 
 // Geometry of output tile `tile` in a merge pass over runs of length w: the

@@ -120,12 +120,12 @@ def test_permute_sort_windows(lib, co, U, pattern):
 
 @pytest.mark.parametrize("U", [5, 1023, 8191, 8193, 3 * 8192 + 1])
 @pytest.mark.parametrize("pattern", ["signed", "signed_wide", "three_groups", "packed", "powers", "groups_of_many", "late_tie",
-                                     "two_ends"])
+                                     "two_ends", "levels"])
 def test_permute_sort_bit_choices(lib, co, U, pattern):
     """Columns for every way in which a tile finds the bits that order its keys: signed numbers
     (small and 100 bits), three far groups, packed bytes and two values (few differing bits),
-    powers of two (lengths), many lengths with long rests (all bits in turn), and a tie in the
-    window that no two neighbours of the input show."""
+    powers of two (lengths), many lengths with long rests or with several levels of ties (further
+    rounds of ranks), and a tie in the window that no two neighbours of the input show."""
     from halo2_amd import device as dv
     from halo2_amd.fields import R_MOD, mont_limbs
     from halo2_amd.lookup import permute_expression_pair_device
@@ -145,6 +145,9 @@ def test_permute_sort_bit_choices(lib, co, U, pattern):
         vals = [1 << (v % 254) for v in wide(16)]
     elif pattern == "groups_of_many":
         vals = [(1 << (253 - v % 40)) + w for v, w in zip(wide(16), wide(100))]
+    elif pattern == "levels":
+        b, c = wide(60)[:3], wide(60)[:3]
+        vals = [(1 << (253 - v % 40)) + (b[v >> 6 & 1] << 100) + (c[v >> 7 & 1] << 20) + (v >> 8 & 3) for v in wide(16)]
     elif pattern == "late_tie":
         vals = wide(253)
         vals[0], vals[-1], vals[U // 2] = vals[1] ^ 5, vals[1] ^ 3, vals[1] ^ (1 << 150)
