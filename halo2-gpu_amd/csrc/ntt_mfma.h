@@ -13,7 +13,7 @@
 // 32 cycles per 64 outputs, after the even/odd split below; leaving them out of a 2^24
 // transform saves 3% of its time). What bounds a step now is the vector unit's issue: ~430
 // instructions per element at ~4 cycles per wave. Coset transforms, against the radix-4 form:
-// 2^16 x 9 125 -> 105 us, 2^20 0.20 -> 0.154 ms, 2^22 0.65 -> 0.55 ms, 2^24 2.60 -> 2.41 ms
+// 2^16 x 9 125 -> 103 us, 2^20 0.165 -> 0.147 ms, 2^22 0.60 -> 0.55 ms, 2^24 2.60 -> 2.40 ms
 // (0.78 ms of it the loads and stores of columns 128 KiB apart).
 //
 // Digits: the matrix columns are the centred residues (|v| <= m/2) in balanced digits
